@@ -108,9 +108,11 @@ int tq4_build_pair_lut(const float *centroids, float *pair_lut, int n_centroids,
 
 /*
  * Full decode step: rotate query into q_rot_ws, build the pair LUT into
- * pair_lut_ws (512 floats), Stage1 into mid_o, Stage2 into out / lse; sinks as in
- * tq4_stage1_ex (may be NULL).  q_rot_ws, pair_lut_ws and mid_o are workspaces: when
- * every (sequence, kv-head) gets one Stage1 wave the step runs one split per sequence and
+ * pair_lut_ws (512 floats), Stage1 into mid_o, merge into out / lse; sinks as in
+ * tq4_stage1_ex (may be NULL).  q_rot_ws, pair_lut_ws and mid_o (B*Hq*num_kv_splits*(D+1)
+ * floats) are workspaces, their contents after the call unspecified: on the 16x16x32 kernel
+ * mid_o holds one row per Stage1 wave (at most num_kv_splits per sequence and head) in a
+ * layout of its own instead of one per split.  When every (sequence, kv-head) gets one wave,
  * Stage1 writes out / lse itself (mid_o unwritten), and for TQ4_BF16 / TQ4_F16 queries with
  * Hk * (waves per kv-head) dividing 8 the same launch also rotates the query (q_rot_ws and
  * pair_lut_ws unwritten).
@@ -130,7 +132,7 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
  * Stage1 rows live in a 40 MiB device array the library holds on every GPU it runs on (from
  * its load until the process ends), so the call allocates nothing -- no hipMalloc, no
  * allocator.  Shapes whose workspace exceeds the array (2 KiB LUT + B*Hq*D*4 bytes of
- * q_rot + B*Hq*S*(D+1)*4 bytes of Stage1 rows unless one split per sequence applies) are
+ * q_rot + B*Hq*S*(D+1)*4 bytes of Stage1 rows unless every sequence gets one wave) are
  * rejected with TQ4_E_INVALID.  Calls that overlap on one GPU share the array and race:
  * serialize them (one stream, or events).  Otherwise as tq4_full_decode.
  * No counterpart in the reference: for callers that cannot allocate (code under graph

@@ -514,24 +514,30 @@ struct Deal {
     int len;         // seq_lens[b], as the deal read it
 };
 
-// Live splits and estimated stream positions of a sequence of len tokens (sequence bb, 0
-// past the batch): each split's tiles (one more when it straddles a tile edge), as the
-// stream pads them.
+// The units dealt and the estimated stream positions of a sequence of len tokens (sequence
+// bb, 0 past the batch).  PARTS: the units are its 16-token tiles, one position each; else its
+// live splits, each with its tiles (one more when it straddles a tile edge), as the stream
+// pads them.
 struct SeqLoad {
     int live;
     uint32_t est;
     int len;
-    int per;  // estimated positions per split
+    int per;  // estimated positions per unit
 };
-__device__ __forceinline__ SeqLoad sequence_load_len(int len, int S) {
+template <bool PARTS> __device__ __forceinline__ SeqLoad sequence_load_len(int len, int S) {
     len = max(len, 0);
+    if constexpr (PARTS) {
+        const int tiles = (len + 15) >> 4;
+        return SeqLoad{tiles, (uint32_t)tiles, len, 1};
+    }
     const int split_len = div_pos(len + S - 1, S);
     const int live = split_len > 0 ? (len + split_len - 1) / split_len : 0;
     const int per = ((split_len + 15) >> 4) + 1;
     return SeqLoad{live, (uint32_t)live * (uint32_t)per, len, per};
 }
+template <bool PARTS>
 __device__ __forceinline__ SeqLoad sequence_load(const int32_t *__restrict__ seq_lens, int B, int S, int bb) {
-    return sequence_load_len(bb < B ? seq_lens[bb] : 0, S);
+    return sequence_load_len<PARTS>(bb < B ? seq_lens[bb] : 0, S);
 }
 
 // Inclusive prefix sum over the wave's 64 lanes: shifts within each 16-lane row, then the
@@ -570,8 +576,8 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // by bisection on its load (lane-wide counts of the waves at least that heavy), then by its
 // place among the waves of exactly that load.  Any x -> p bijection keeps the deal exact.
 // lane_len: seq_lens[lane] (0 past the batch), read by the caller.
-__device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane) {
-    const SeqLoad q = sequence_load_len(lane_len, S);
+template <bool PARTS> __device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane) {
+    const SeqLoad q = sequence_load_len<PARTS>(lane_len, S);
     const uint32_t est_total = wave_sum(q.est);
     const int n_live = __builtin_popcountll(__ballot(q.live > 0));
     // spare waves before prefix pre: floor(pre * spare / total) with one fp32 ratio -- monotone
@@ -579,10 +585,10 @@ __device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane)
     const float ratio = est_total > 0 ? (float)((int64_t)nw * B - n_live) / (float)est_total : 0.f;
     auto cut = [&](uint32_t pre) { return (int)floorf((float)pre * ratio); };
     const uint32_t est_out = wave_scan(q.est);
-    const int k = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), q.live) : 0;
-    const int per = q.live > 0 ? q.per : 0;  // positions per split
-    // live / k and live % k: an fp32 quotient is within 1 of it for live below 2^22 (live <= S),
-    // so one correction step makes it exact
+    const int k = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), PARTS ? min(q.live, S) : q.live) : 0;
+    const int per = q.live > 0 ? q.per : 0;  // positions per unit
+    // live / k and live % k: an fp32 quotient is within 1 of it for live below 2^22 (live <= S;
+    // PARTS: 2^22 tiles are 2^26 tokens), so one correction step makes it exact
     int qd = 0, r = 0;
     if (k > 0) {
         qd = (int)((float)q.live * __builtin_amdgcn_rcpf((float)k));
@@ -624,6 +630,7 @@ __device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane)
     return Deal{sq, j, __builtin_amdgcn_readlane(k, sq), __builtin_amdgcn_readlane(q.len, sq)};
 }
 
+template <bool PARTS>
 __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, int nw, int x, int lane) {
     // equal lengths: every sequence keeps its nw waves, as the deal would give them
     const int len0 = seq_lens[0];
@@ -639,12 +646,12 @@ __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, i
     if (equal)
         return Deal{x / nw, x % nw, nw, len0};
     if (B <= kWave)
-        return deal_ranked(lane_len, B, S, nw, x, lane);
-    const SeqLoad first = sequence_load_len(lane_len, S);
+        return deal_ranked<PARTS>(lane_len, B, S, nw, x, lane);
+    const SeqLoad first = sequence_load_len<PARTS>(lane_len, S);
     uint32_t est_total = 0;
     int n_live = 0;
     for (int c0 = 0; c0 < B; c0 += kWave) {
-        const SeqLoad q = c0 == 0 ? first : sequence_load(seq_lens, B, S, c0 + lane);
+        const SeqLoad q = c0 == 0 ? first : sequence_load<PARTS>(seq_lens, B, S, c0 + lane);
         est_total += (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(q.est), kWave - 1);
         n_live += __builtin_popcountll(__ballot(q.live > 0));
     }
@@ -655,9 +662,10 @@ __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, i
     uint32_t est_carry = 0;
     int wave_carry = 0;
     for (int c0 = 0; c0 < B; c0 += kWave) {
-        const SeqLoad q = c0 == 0 ? first : sequence_load(seq_lens, B, S, c0 + lane);
+        const SeqLoad q = c0 == 0 ? first : sequence_load<PARTS>(seq_lens, B, S, c0 + lane);
         const uint32_t est_out = est_carry + wave_scan(q.est);
-        const int mine = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), q.live) : 0;
+        const int mine =
+            q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), PARTS ? min(q.live, S) : q.live) : 0;
         const int w_out = wave_carry + (int)wave_scan((uint32_t)mine);
         const int w_in = w_out - mine;
         const uint64_t hit = __ballot(x >= w_in && x < w_out);
@@ -1149,12 +1157,12 @@ __device__ __forceinline__ void put_out(void *out, int dtype, int64_t i, float v
 // exp(0) = 1, sum 1), so the wave writes the final output rows and LSE itself -- the same
 // values Stage2 would write, without the mid_o round trip.
 // Heads nh .. G-1 of the wave are padding (a GQA group that is not a multiple of G).
-template <int G>
+template <int G, bool V3>
 __device__ __forceinline__ void emit_output(const State &st, const floatx4 (&acc)[8], const LaneConst &lc,
                                             void *out, int out_dtype, float *lse, int64_t row0, int nh) {
     int h0;
     float o[G / 4][8], safe_l;
-    finish_rows<G, false>(st, acc, lc, h0, o, safe_l);
+    finish_rows<G, V3>(st, acc, lc, h0, o, safe_l);
     const int64_t r = (row0 + h0) * kHeadDim + 8 * lc.n;
 #pragma unroll
     for (int k = 0; k < G / 4; ++k)
@@ -1164,6 +1172,31 @@ __device__ __forceinline__ void emit_output(const State &st, const floatx4 (&acc
                 put_out(out, out_dtype, r + k * kHeadDim + i, o[k][i]);
     if (lc.g == 0 && lc.n < nh)
         lse[row0 + lc.n] = lse_of(st.negm, safe_l);
+}
+
+// Row `wid` of each head's part rows: the wave's outputs and LSE, and, from the sequence's
+// first wave, how many rows there are (layout: part_rows / part_lse in stage2.h).
+template <int G, bool V3>
+__device__ __forceinline__ void emit_part(const State &st, const floatx4 (&acc)[8], const LaneConst &lc,
+                                          float *__restrict__ parts, int64_t total_rows, int64_t row0, int num_splits,
+                                          int wid, int run_waves, int nh) {
+    int h0;
+    float o[G / 4][8], safe_l;
+    finish_rows<G, V3>(st, acc, lc, h0, o, safe_l);
+    typedef float float4a __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for (int k = 0; k < G / 4; ++k)
+        if (h0 + k < nh) {
+            float *r = part_row(parts, row0 + h0 + k, num_splits, wid) + 8 * lc.n;
+            *reinterpret_cast<float4a *>(r) = float4a{o[k][0], o[k][1], o[k][2], o[k][3]};
+            *reinterpret_cast<float4a *>(r + 4) = float4a{o[k][4], o[k][5], o[k][6], o[k][7]};
+        }
+    if (lc.g == 0 && lc.n < nh) {
+        float *l = part_lse(parts, total_rows, row0 + lc.n, num_splits);
+        l[wid] = part_lse_value(lse_of(st.negm, safe_l));
+        if (wid == 0 && run_waves < num_splits)
+            l[num_splits - 1] = part_count_mark(run_waves);
+    }
 }
 
 // Write image slots 0 .. ns-1 to the rows of splits s0 .. s0+ns-1 (heads 0 .. nh-1; the
@@ -1313,14 +1346,22 @@ __device__ __forceinline__ void rot_column_tile(const half8 (&ah)[G / 2][4], con
 // nh .. G-1 as padding (zero queries, never written).  Grid x runs over the (part, kv-head)
 // pairs, vh = part * Hk + kv-head.
 //
-// FUSED (launched with one split per sequence and one wave per (sequence, kv-head part)): the
-// wave writes the final output rows (out, out_dtype) and LSE instead of mid_o rows.
-// ROT (with FUSED; 1: bf16 queries, 2: fp16): a workgroup is the nvh waves of one sequence
+// PARTS (the full decode step, whose split rows nobody else reads): no splits.  A sequence's
+// 16-token tiles are divided among its waves, each wave takes one contiguous run of them and
+// leaves one row per head (mid_o in the layout of part_row, stage2.h; merged by
+// merge_parts_kernel).  Against num_splits rows this drops the mid_o traffic of all but one
+// row per wave, the split ends inside the stream, and, for lengths that are not a multiple of
+// 16 num_splits, the tiles that two splits share and the padding of each split.  With one
+// wave per (sequence, kv-head part) (gridDim.y = 1) that wave owns the whole sequence and
+// writes the final output rows (out, out_dtype) and LSE itself.
+// Measured, full step with 32 splits, B64 x 32/8 heads: 4096 tokens 82.6 -> 68.8 us (AoS 97.1 ->
+// 84.2), ragged 512..8192 95.3 -> 77.3.
+// ROT (with PARTS; 1: bf16 queries, 2: fp16): a workgroup is the nvh waves of one sequence
 // (grid (B)), which rotate the query themselves (q_rot is not read: `query`, `rot_t`, and
 // pair_lut holds the 16 centroids).
 // KF8: the FP8-key preset (K one E4M3 byte per dim, no norm, the query not rotated).
 // KB3: the 3-bit-key / 4-bit-value preset (pair_lut then holds the 8 centroids).
-template <int LAYOUT, int G, int WPE, bool FUSED, bool KF8 = false, bool KB3 = false, bool V3 = false, int ROT = 0>
+template <int LAYOUT, int G, int WPE, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false, int ROT = 0>
 __global__ __launch_bounds__(ROT ? kWave * kRotGroupWaves : kWave) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void stage1_xdl_kernel(
     const float *__restrict__ q_rot, const uint8_t *__restrict__ cache,
@@ -1331,7 +1372,7 @@ void stage1_xdl_kernel(
     int slot_pos, int slot_head, int num_splits, float score_scale_log2,
     const void *__restrict__ query, const float *__restrict__ rot_t) {
     static_assert(G == 4 || G == 8, "4 or 8 q-heads per wave");
-    static_assert(ROT == 0 || (FUSED && !KF8 && !KB3), "the query rotation runs in the one-split 4-bit kernel");
+    static_assert(ROT == 0 || (PARTS && !KF8 && !KB3), "the query rotation runs in the one-wave 4-bit kernel");
     using QueryT = std::conditional_t<ROT == 1, __bf16, _Float16>;
     constexpr int TPL = G / 4;
     constexpr int RING = 4;
@@ -1391,12 +1432,20 @@ void stage1_xdl_kernel(
     // lengths make right.  When the first chunk's entries turn out to be exactly these, the
     // registers serve it and the block-table read leaves the path to the first KV loads;
     // otherwise the guess has warmed L2 for the real reads.
-    const int guess_b = b, guess_first = wid * ((max_blocks + nw - 1) / nw);
-    const int bt_guess = block_table[(int64_t)b * max_blocks + min(guess_first + lane, max_blocks - 1)];
+    const int guess_b = b;
+    int guess_block, guess_tile = 0;  // lane i: the block of the guessed run's tile i (PARTS: from guess_tile)
+    if constexpr (PARTS) {
+        const int tl = block_size_log2 - 4, most = max_blocks << tl, q = most / nw;
+        guess_tile = wid * q + min(wid, most - q * nw);
+        guess_block = min((guess_tile + lane) >> tl, max_blocks - 1);
+    } else {
+        guess_block = min(wid * ((max_blocks + nw - 1) / nw) + lane, max_blocks - 1);
+    }
+    const int bt_guess = block_table[(int64_t)b * max_blocks + guess_block];
     // The pair-LUT rows do not depend on the sequence: they go out first; the K table and the
     // q operands are built once the first tiles' loads are on their way.
     static_assert(!(KF8 && KB3), "one key format");
-    static_assert(!V3 || (KB3 && !FUSED), "3-bit values come with 3-bit keys, not fused");
+    static_assert(!V3 || KB3, "3-bit values come with 3-bit keys");
     // 3-bit presets, SoA: records staged through LDS (RawRec), see stage_records
     constexpr bool STG = KB3 && LAYOUT == 0;
     // FP8 keys, SoA: records staged the same way (RawRec3)
@@ -1418,26 +1467,33 @@ void stage1_xdl_kernel(
     const float sink = *(sinks ? sinks + hb + hl : q_rot);
     int run_waves = nw;  // waves sharing this wave's sequence and kv-head
     int dealt_len = 0;
-    if constexpr (!FUSED) {
-        const Deal d = deal_waves(seq_lens, gridDim.z, num_splits, nw, wid + nw * b, lane);
+    const bool whole = PARTS && nw == 1;  // the wave owns its sequence (of this kv-head part)
+    if (ROT || whole) {
+        dealt_len = seq_lens[b];
+    } else {
+        const Deal d = deal_waves<PARTS>(seq_lens, gridDim.z, num_splits, nw, wid + nw * b, lane);
         if (d.b < 0)
             return;
         b = d.b;
         wid = d.wid;
         run_waves = d.nw;
         dealt_len = d.len;
+        if (PARTS)  // equal lengths: every sequence is dealt nw waves, at most one per tile
+            run_waves = min(run_waves, (max(dealt_len, 0) + 15) >> 4);
     }
-    const int seq_len = FUSED ? seq_lens[b] : dealt_len;
-    // split partition: L = ceil(len / S); live splits are those with s * L < len
-    const int split_len = div_pos(max(seq_len, 0) + num_splits - 1, num_splits);
-    const int live = split_len > 0 ? min(num_splits, div_pos(seq_len + split_len - 1, split_len)) : 0;
+    const int seq_len = dealt_len;
+    // split partition: L = ceil(len / S); live splits are those with s * L < len.  PARTS: the
+    // "splits" are the 16-token tiles, of which the wave's run makes one row
+    const int split_len = PARTS ? 16 : div_pos(max(seq_len, 0) + num_splits - 1, num_splits);
+    const int live = PARTS ? (max(seq_len, 0) + 15) >> 4
+                           : split_len > 0 ? min(num_splits, div_pos(seq_len + split_len - 1, split_len)) : 0;
     // run x of the W runs of this (sequence, kv-head): live splits from x q + min(x, r), q + 1 of
     // them for x < r and q after (q = live / W, r = live % W)
-    const int run_q = div_pos(live, run_waves), run_r = live - run_q * run_waves;
+    const int run_q = PARTS && run_waves <= 0 ? 0 : div_pos(live, run_waves), run_r = live - run_q * run_waves;
     const int s_lo = wid * run_q + min(wid, run_r);
-    const int s_hi = s_lo + run_q + (wid < run_r ? 1 : 0);
-    if constexpr (FUSED) {
-        if (live == 0) {
+    const int s_hi = wid < run_waves ? s_lo + run_q + (wid < run_r ? 1 : 0) : s_lo;
+    if constexpr (PARTS) {
+        if (whole && live == 0) {
             // an empty sequence: what Stage2 writes for it (0 / 0 and ln 0); with ROT every
             // wave of the workgroup returns here (one sequence), before its barrier
             const int64_t r0 = ((int64_t)b * num_q_heads + hb) * kHeadDim;
@@ -1466,11 +1522,10 @@ void stage1_xdl_kernel(
     constexpr int kRec = record_bytes<LAYOUT, KF8, KB3, V3>();
     constexpr int kStage = STG ? 16 * kRec + 16 : STG8 ? 16 * kRec : 0;
     __shared__ __align__(16) uint8_t recbuf[kStage > 0 ? kStage : 16];
-    // split starts of a chunk, one byte per stream position (chunk_tiles; one split per wave
-    // when FUSED)
-    __shared__ uint8_t marks[FUSED ? 1 : kWave];
-    using Cap = SpanCap<LAYOUT, G, WPE, (KF8 ? 0 : KTable<LAYOUT>::words * 4) + kStage + (FUSED ? 0 : kWave)>;
-    __shared__ __align__(16) float img[FUSED ? 4 : Cap::floats];  // FUSED writes no mid_o rows
+    // split starts of a chunk, one byte per stream position (chunk_tiles; PARTS has no splits)
+    __shared__ uint8_t marks[PARTS ? 1 : kWave];
+    using Cap = SpanCap<LAYOUT, G, WPE, (KF8 ? 0 : KTable<LAYOUT>::words * 4) + kStage + (PARTS ? 0 : kWave)>;
+    __shared__ __align__(16) float img[PARTS ? 4 : Cap::floats];  // PARTS: rows go out from registers
     __shared__ __align__(16) float qbuf[ROT ? kRotGroupWaves * G * kQRowFloats : 4];
     half8 bq[8];
     float q_unscale = 1.f;  // 2^-e of the lane's q row (q_operands)
@@ -1503,7 +1558,9 @@ void stage1_xdl_kernel(
     int sp_tf = 0, sp_nt = 0, sp_base = 0;
     int e_log2 = -1;  // log2 of the positions of every split of the run when they are one power of two
     int total = 0;
-    if (run_in_lanes) {
+    if constexpr (PARTS) {
+        total = n_run;
+    } else if (run_in_lanes) {
         const int st0 = (s_lo + min(lane, n_run - 1)) * split_len, en = min(st0 + split_len, seq_len);
         sp_tf = st0 >> 4;
         sp_nt = ((en - 1) >> 4) - sp_tf + 1;
@@ -1532,8 +1589,8 @@ void stage1_xdl_kernel(
     int cur = s_lo;
     int img_s0 = s_lo;  // split of image slot 0
     int cur_start = cur * split_len;
-    int cur_end = min(cur_start + split_len, seq_len);
-    int cur_stop = split_stop(cur);
+    int cur_end = min(PARTS ? 16 * s_hi : cur_start + split_len, seq_len);
+    int cur_stop = PARTS ? 0 : split_stop(cur);
 
     // Lane i of base_lo / base_hi holds the address of the 16-token piece at stream
     // position j0 + i of the current chunk (its KV block plus the piece's offset), lane i
@@ -1646,7 +1703,11 @@ void stage1_xdl_kernel(
     // Lane i: the tile and mask of stream position j0 + i and the block-table entry of that
     // tile (read here; the addresses come from chunk_addresses).
     auto chunk_tiles = [&](int j0, int nchunk) {
-        if (run_in_lanes && e_log2 >= 0) {
+        if constexpr (PARTS) {
+            const int p = j0 + min(lane, nchunk - 1);
+            tile_lane = s_lo + min(p, n_run - 1);
+            mask_lane = p < n_run ? tile_lane : -(1 << 24);  // padding: no valid token
+        } else if (run_in_lanes && e_log2 >= 0) {
             // every split takes 2^e_log2 positions (the tail's go to the last one)
             const int p = j0 + min(lane, nchunk - 1);
             const int i = min(p >> e_log2, n_run - 1);
@@ -1656,21 +1717,19 @@ void stage1_xdl_kernel(
             mask_lane = o < nt ? tile_lane : -(1 << 24);  // padding: no valid token
         } else if (run_in_lanes) {
             int i = 0;  // the lane's split, as an index into the run
-            if constexpr (!FUSED) {
-                if (n_run > 1) {
-                    // the splits that start inside (j0, j0 + 64) mark their offset; position
-                    // j0 + q lies in the split that holds j0, moved on by the marks up to q
-                    marks[lane] = 0;
-                    const int q = sp_base - j0;
-                    if (lane < n_run && q > 0 && q < kWave)
-                        marks[q] = 1;
-                    // other lanes' marks: the compiler must not forward the lane's own stores
-                    // (one wave: its LDS writes complete before its later reads)
-                    asm volatile("" ::: "memory");
-                    const uint64_t m = __ballot(marks[lane] != 0);
-                    const int i0 = __builtin_popcountll(__ballot(lane < n_run && sp_base <= j0)) - 1;
-                    i = __shfl(i0 + __builtin_popcountll(m & (~0ull >> (63 - lane))), min(lane, nchunk - 1), kWave);
-                }
+            if (n_run > 1) {
+                // the splits that start inside (j0, j0 + 64) mark their offset; position
+                // j0 + q lies in the split that holds j0, moved on by the marks up to q
+                marks[lane] = 0;
+                const int q = sp_base - j0;
+                if (lane < n_run && q > 0 && q < kWave)
+                    marks[q] = 1;
+                // other lanes' marks: the compiler must not forward the lane's own stores
+                // (one wave: its LDS writes complete before its later reads)
+                asm volatile("" ::: "memory");
+                const uint64_t m = __ballot(marks[lane] != 0);
+                const int i0 = __builtin_popcountll(__ballot(lane < n_run && sp_base <= j0)) - 1;
+                i = __shfl(i0 + __builtin_popcountll(m & (~0ull >> (63 - lane))), min(lane, nchunk - 1), kWave);
             }
             const int o = j0 + min(lane, nchunk - 1) - __shfl(sp_base, i, kWave);
             const int nt = __shfl(sp_nt, i, kWave);
@@ -1693,8 +1752,13 @@ void stage1_xdl_kernel(
             }
         }
         const int bidx = (16 * tile_lane) >> block_size_log2;
-        const bool guessed = j0 == 0 && b == guess_b &&
-                             __ballot(bidx != min(guess_first + lane, max_blocks - 1)) == 0;
+        if constexpr (PARTS) {
+            // the run starts where the guess did: lane i of the guess holds tile i's block
+            if (j0 == 0 && b == guess_b && s_lo == guess_tile)
+                return __shfl(bt_guess, tile_lane - s_lo, kWave);
+            return bt[bidx];
+        }
+        const bool guessed = j0 == 0 && b == guess_b && __ballot(bidx != guess_block) == 0;
         return guessed ? bt_guess : bt[bidx];
     };
     auto chunk_addresses = [&](int blk) {
@@ -1811,9 +1875,9 @@ void stage1_xdl_kernel(
                 if (k & 1) {
                     issue_vpos(vr[k - 1], pos[(k + 3) % RING], moff_lane, min(j + k - 1 + RING, last));
                     issue_vpos(vr[k], pos[k % RING], moff_lane, min(j + k + RING, last));
-                    // a split ends after an odd stage (FUSED: the only split ends with the
-                    // stream; its rows are written after the loop)
-                    if (!FUSED && j + k + 1 == pos_base + cur_stop) {
+                    // a split ends after an odd stage (PARTS: the one row ends with the
+                    // stream and is written after the loop)
+                    if (!PARTS && j + k + 1 == pos_base + cur_stop) {
                         stash_split<G, Cap, V3>(st, acc, lc, img, cur - img_s0);
                         if (cur + 1 == s_hi || cur + 1 - img_s0 == Cap::splits) {
                             flush_splits<G, Cap>(img, mid_o, row0, num_splits, img_s0, cur + 1 - img_s0, lane, nh);
@@ -1835,8 +1899,13 @@ void stage1_xdl_kernel(
             j += RING;
         } while (j <= last);
     }
-    if constexpr (FUSED)
-        emit_output<G>(st, acc, lc, out, out_dtype, lse, row0, nh);
+    if constexpr (PARTS) {
+        if (ROT || whole)
+            emit_output<G, V3>(st, acc, lc, out, out_dtype, lse, row0, nh);
+        else
+            emit_part<G, V3>(st, acc, lc, mid_o, (int64_t)gridDim.z * num_q_heads, row0, num_splits, wid, run_waves,
+                             nh);
+    }
 }
 
 }  // namespace xdl

@@ -91,6 +91,80 @@ __global__ __launch_bounds__(kWave) void stage2_kernel(const float *__restrict__
         lse[(int64_t)b * num_q_heads + h] = mx + logf(wsum);
 }
 
+// ---- Part rows: what Stage1 leaves when it runs a full decode step ----------------------
+// Inside the step nobody but the merge reads Stage1's rows, so mid_o's num_splits * 129
+// floats per (sequence, head) row hold `parts <= num_splits` rows in a layout of their own:
+// all rows' 128 outputs first (part p of row r at (r * num_splits + p) * 128), then all LSEs
+// (r * num_splits + p).  `parts` is worked out inside Stage1 (one per wave dealt to the
+// sequence); when it is below num_splits the last LSE slot, then unused, holds it as a NaN
+// with all sign, exponent and quiet bits set, which no stored LSE has.
+__device__ __forceinline__ float *part_row(float *parts, int64_t row, int num_splits, int p) {
+    return parts + (row * num_splits + p) * kHeadDim;
+}
+__device__ __forceinline__ float *part_lse(float *parts, int64_t total_rows, int64_t row, int num_splits) {
+    return parts + total_rows * num_splits * kHeadDim + row * num_splits;
+}
+constexpr uint32_t kPartMark = 0xFFC00000u;
+__device__ __forceinline__ float part_count_mark(int n) { return __builtin_bit_cast(float, kPartMark | (uint32_t)n); }
+__device__ __forceinline__ float part_lse_value(float x) { return x != x ? __builtin_nanf("") : x; }
+
+// One wave per (q-head, sequence): out = sum_p w_p o_p / sum_p w_p, w_p = exp(lse_p - max), as
+// stage2_kernel; lane owns dims 2 lane, 2 lane + 1.  Bound by latency (B64 x 32 heads x 4
+// parts are 4 MB): the length, the count, the LSEs and the first CHUNK rows are all requested
+// at once (rows past the count are in bounds, and replaced by zeros with weight 0).
+template <typename OutT, int CHUNK>
+__global__ __launch_bounds__(kWave) void merge_parts_kernel(const float *__restrict__ parts,
+                                                           const int32_t *__restrict__ seq_lens,
+                                                           OutT *__restrict__ out, float *__restrict__ lse,
+                                                           int num_q_heads, int num_splits) {
+    const int b = blockIdx.y, lane = threadIdx.x;
+    const int64_t row = (int64_t)b * num_q_heads + blockIdx.x;
+    const int64_t total_rows = (int64_t)gridDim.y * num_q_heads;
+    typedef float float2a __attribute__((ext_vector_type(2), aligned(4)));
+    const float *r = part_row(const_cast<float *>(parts), row, num_splits, 0) + 2 * lane;
+    const float *lr = part_lse(const_cast<float *>(parts), total_rows, row, num_splits);
+    float l;
+    float2a v[CHUNK];
+    auto load_chunk = [&](int s0, int n_rows) {
+        l = lr[s0 + min(lane, n_rows - 1)];
+#pragma unroll
+        for (int i = 0; i < CHUNK; ++i)
+            v[i] = *reinterpret_cast<const float2a *>(r + (int64_t)(s0 + min(i, n_rows - 1)) * kHeadDim);
+    };
+    load_chunk(0, min(CHUNK, num_splits));
+    const uint32_t mark = __builtin_bit_cast(uint32_t, lr[num_splits - 1]);
+    const int seq_len = seq_lens[b];
+    int n_parts = (mark & kPartMark) == kPartMark ? (int)(mark & ~kPartMark) : num_splits;
+    n_parts = seq_len > 0 ? min(n_parts, num_splits) : 0;  // an empty sequence wrote nothing
+
+    float mx = -INFINITY, a0 = 0.f, a1 = 0.f, wsum = 0.f;
+    for (int s0 = 0; s0 < n_parts; s0 += CHUNK) {
+        const int n = min(CHUNK, n_parts - s0);
+        if (s0 > 0)
+            load_chunk(s0, n);
+        l = lane < n ? l : -INFINITY;
+        const float m_new = fmaxf(mx, wave_max(l));
+        const float scale = expf(mx - m_new);  // 0 for the first chunk (mx = -inf)
+        const float w = expf(l - m_new);       // 0 on lanes past the chunk
+        a0 *= scale;
+        a1 *= scale;
+        wsum = wsum * scale + wave_sum(w);
+#pragma unroll
+        for (int i = 0; i < CHUNK; ++i) {
+            const float wi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), i));
+            a0 = fmaf(wi, i < n ? v[i][0] : 0.f, a0);
+            a1 = fmaf(wi, i < n ? v[i][1] : 0.f, a1);
+        }
+        mx = m_new;
+    }
+    const float inv = 1.f / wsum;
+    OutT *o = out + row * kHeadDim;
+    o[2 * lane] = from_float<OutT>(a0 * inv);
+    o[2 * lane + 1] = from_float<OutT>(a1 * inv);
+    if (lane == 0)
+        lse[row] = mx + logf(wsum);
+}
+
 // Rotation on the f16 matrix cores: q_rot = query @ rot_t with rot_t split into f16
 // hi + lo parts (hi + lo = rot_t to ~2^-22), and for fp32 queries the query too
 // (products hi*hi + hi*lo + lo*hi).  Each query row is first scaled by a power of two 2^e

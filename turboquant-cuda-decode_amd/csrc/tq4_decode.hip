@@ -6,6 +6,7 @@
 // message instead of throwing.
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
+#include <algorithm>
 #include <atomic>
 #include <cstdarg>
 #include <mutex>
@@ -82,7 +83,8 @@ struct Stage1Args {
     int S, layout;  // TQ4_LAYOUT_*
     float scale;
     const float *sinks = nullptr;  // [Hq] sink logits of split 0, or null
-    // set: one split per sequence, the XDL kernel writes the final rows (Stage2 fused)
+    // set: a full decode step on the XDL kernel (PARTS): part rows in mid_o, or with one wave
+    // per (sequence, kv-head part) the final rows
     void *out = nullptr;
     int out_dtype = TQ4_F32;
     float *lse = nullptr;
@@ -192,7 +194,7 @@ int xdl_parts(const Stage1Args &a) {
 // whole rounds of the waves the GPU holds at the kernel's occupancy.  `slots` caches that
 // count per kernel instance (computed on the first call; concurrent first calls compute the
 // same value).  TQ4_STAGE1_WAVES overrides W (a tuning knob; results do not depend on it).
-int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int> &slots) {
+int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int> &slots, int per_simd) {
     static const int forced = [] {
         const char *e = getenv("TQ4_STAGE1_WAVES");
         return e ? atoi(e) : 0;
@@ -206,7 +208,7 @@ int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int>
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tq4::kWave, 0) == hipSuccess &&
             cus > 0 && per_cu > 0)
-            held = cus * per_cu;
+            held = cus * std::min(per_cu, 4 * per_simd);
         else
             held = 256 * 4 * 2;
         slots.store(held, std::memory_order_relaxed);
@@ -229,10 +231,23 @@ template <int LAYOUT, int G> constexpr int xdl_waves_per_simd() {
     return LAYOUT == 0 && G == 4 ? TQ4_XDL_WAVES_PER_SIMD : 2;
 }
 
-template <int LAYOUT, int G, bool KF8 = false, bool KB3 = false, bool V3 = false> int xdl_waves(const Stage1Args &a) {
+// The kernel of one key / value format; PARTS: the full decode step's form of it.
+template <int LAYOUT, int G, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false> constexpr auto xdl_kernel() {
+    return &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, xdl_waves_per_simd<LAYOUT, G>(), PARTS, KF8, KB3, V3>;
+}
+template <int LAYOUT, int G, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false>
+int xdl_waves(const Stage1Args &a) {
     static std::atomic<int> slots{0};
-    const auto kernel = &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, xdl_waves_per_simd<LAYOUT, G>(), false, KF8, KB3, V3>;
-    return waves_per_sequence(a, reinterpret_cast<const void *>(kernel), slots);
+    return waves_per_sequence(a, reinterpret_cast<const void *>(xdl_kernel<LAYOUT, G, PARTS, KF8, KB3, V3>()), slots,
+                              xdl_waves_per_simd<LAYOUT, G>());
+}
+template <int LAYOUT, int G, bool PARTS> int xdl_waves_of(const Stage1Args &a) {
+    if (a.key_fp8)
+        return xdl_waves<LAYOUT, G, PARTS, true>(a);
+    if (a.key_bits == 3)
+        return a.value_bits == 3 ? xdl_waves<LAYOUT, G, PARTS, false, true, true>(a)
+                                 : xdl_waves<LAYOUT, G, PARTS, false, true>(a);
+    return xdl_waves<LAYOUT, G, PARTS>(a);
 }
 
 // The one-split kernel that rotates the query itself: one workgroup per sequence holding its
@@ -244,7 +259,6 @@ bool rot_applies(const Stage1Args &a) {
 
 template <int LAYOUT, int G> void launch_xdl(const Stage1Args &a, hipStream_t st) {
     constexpr int wpe = xdl_waves_per_simd<LAYOUT, G>();
-    const bool kb3 = a.key_bits == 3, v3 = a.value_bits == 3;
     const int nvh = a.Hk * xdl_parts(a);
     if (a.query) {  // one split per sequence, the rotation inside (Stage2 fused)
         const auto kernel = a.query_dtype == TQ4_BF16
@@ -255,17 +269,14 @@ template <int LAYOUT, int G> void launch_xdl(const Stage1Args &a, hipStream_t st
                a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, a.query, a.rot_t);
         return;
     }
-    const int waves = a.key_fp8 ? xdl_waves<LAYOUT, G, true>(a)
-                      : kb3     ? (v3 ? xdl_waves<LAYOUT, G, false, true, true>(a) : xdl_waves<LAYOUT, G, false, true>(a))
-                                : xdl_waves<LAYOUT, G>(a);
-    const dim3 grid(nvh, waves, a.B);
-    auto kernel = a.out ? &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, true>
-                        : &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, false>;
-    if (a.key_fp8)  // never fused: the FP8-key decode runs Stage2 itself
-        kernel = &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, false, true>;
-    else if (kb3)  // 3-bit keys, 4- or 3-bit values; never fused
-        kernel = v3 ? &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, false, false, true, true>
-                    : &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, false, false, true>;
+    const dim3 grid(nvh, a.out ? xdl_waves_of<LAYOUT, G, true>(a) : xdl_waves_of<LAYOUT, G, false>(a), a.B);
+    auto kernel = a.out ? xdl_kernel<LAYOUT, G, true>() : xdl_kernel<LAYOUT, G, false>();
+    if (a.key_fp8)
+        kernel = a.out ? xdl_kernel<LAYOUT, G, true, true>() : xdl_kernel<LAYOUT, G, false, true>();
+    else if (a.key_bits == 3 && a.value_bits == 3)
+        kernel = a.out ? xdl_kernel<LAYOUT, G, true, false, true, true>() : xdl_kernel<LAYOUT, G, false, false, true, true>();
+    else if (a.key_bits == 3)
+        kernel = a.out ? xdl_kernel<LAYOUT, G, true, false, true>() : xdl_kernel<LAYOUT, G, false, false, true>();
     launch(kernel, grid, dim3(tq4::kWave), st, a.q_rot, a.cache, a.bt, a.seq_lens, a.lut,
            a.mid_o, a.sinks, a.out, a.out_dtype, a.lse, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks,
            a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, nullptr, nullptr);
@@ -306,15 +317,15 @@ template <int LAYOUT> int dispatch_xdl(const Stage1Args &a, hipStream_t st) {
     return launch_status("stage1_xdl");
 }
 
-// Waves per (sequence, kv-head) the auto Stage1 kernel runs with (0 when it is not the
-// 16x16x32 kernel).
-int auto_xdl_waves(const Stage1Args &a) {
+// Waves per (sequence, kv-head part) of the full decode step (0 when the 16x16x32 kernel does
+// not apply).
+int decode_waves(const Stage1Args &a) {
     if (!mfma_applies(a))
         return 0;
     const bool g4 = xdl_heads(a) == 4;
     if (a.kl == 0)
-        return g4 ? xdl_waves<0, 4>(a) : xdl_waves<0, 8>(a);
-    return g4 ? xdl_waves<1, 4>(a) : xdl_waves<1, 8>(a);
+        return g4 ? xdl_waves_of<0, 4, true>(a) : xdl_waves_of<0, 8, true>(a);
+    return g4 ? xdl_waves_of<1, 4, true>(a) : xdl_waves_of<1, 8, true>(a);
 }
 
 int run_stage1(Stage1Args a, int kernel, hipStream_t st) {
@@ -325,16 +336,12 @@ int run_stage1(Stage1Args a, int kernel, hipStream_t st) {
     if (kernel == TQ4_KERNEL_MFMA)
         return fail(TQ4_E_UNSUPPORTED, "tq4_stage1_ex: the 4x4x4 MFMA kernel is retired; "
                                        "TQ4_KERNEL_XDL (16x16x32) covers the same shapes");
-    if (a.key_fp8 && a.out)
-        return fail(TQ4_E_UNSUPPORTED, "tq4_stage1_fp8: no fused Stage2 for FP8 keys");
     // the bit-width presets: 3-bit K (4- or 3-bit V) also on the 16x16x32 kernel, 4/4 VALU
     const bool preset_xdl = a.key_bits == 3;
     if (a.key_bits > 0 && kernel != TQ4_KERNEL_AUTO && kernel != TQ4_KERNEL_SIMPLE &&
         !(preset_xdl && kernel == TQ4_KERNEL_XDL))
         return fail(TQ4_E_UNSUPPORTED, "tq4_stage1_preset: key/value bits %d/%d run on the VALU kernel%s",
                     a.key_bits, a.value_bits, preset_xdl ? " or the 16x16x32 kernel" : "");
-    if (a.key_bits > 0 && a.out)
-        return fail(TQ4_E_UNSUPPORTED, "tq4_stage1_preset: no fused Stage2 for the bit-width presets");
     if (kernel == TQ4_KERNEL_AUTO)
         kernel = (a.key_bits > 0 && !preset_xdl) ? TQ4_KERNEL_SIMPLE
                                                  : (mfma_applies(a) ? TQ4_KERNEL_XDL : TQ4_KERNEL_SIMPLE);
@@ -343,6 +350,31 @@ int run_stage1(Stage1Args a, int kernel, hipStream_t st) {
     if (kernel == TQ4_KERNEL_XDL)
         return a.kl == 0 ? dispatch_xdl<0>(a, st) : dispatch_xdl<1>(a, st);
     return fail(TQ4_E_INVALID, "tq4_stage1_ex: unknown kernel id %d", kernel);
+}
+
+// Rows the merge requests ahead of the part count: 8 cover what a ragged batch usually deals
+// a sequence at up to 8 waves each (more are read in further chunks of 8), 32 the rest.
+constexpr int kMergeSmall = 8, kMergeLarge = 32;
+
+// The attention of a full decode step from rotated queries: Stage1 in part rows, then their
+// merge; `waves` = decode_waves(a).  With one wave per (sequence, kv-head part) Stage1 writes
+// the output rows itself.
+int run_parts(const Stage1Args &a, int waves, hipStream_t st) {
+    const int rc = run_stage1(a, TQ4_KERNEL_XDL, st);
+    if (rc || waves == 1)
+        return rc;
+    const bool small = waves <= kMergeSmall;
+    const dim3 grid(a.Hq, a.B), block(tq4::kWave);
+#define TQ4_MERGE_LAUNCH(T)                                                                                     \
+    launch(small ? &tq4::merge_parts_kernel<T, kMergeSmall> : &tq4::merge_parts_kernel<T, kMergeLarge>, grid, block, \
+           st, a.mid_o, a.seq_lens, static_cast<T *>(a.out), a.lse, a.Hq, a.S)
+    switch (a.out_dtype) {
+    case TQ4_F32: TQ4_MERGE_LAUNCH(float); break;
+    case TQ4_BF16: TQ4_MERGE_LAUNCH(__bf16); break;
+    default: TQ4_MERGE_LAUNCH(_Float16); break;
+    }
+#undef TQ4_MERGE_LAUNCH
+    return launch_status("merge_parts");
 }
 
 int rotate_query(const void *query, int query_dtype, const float *rot_t, float *q_rot, int rows,
@@ -593,25 +625,20 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
     if (!centroids || !pair_lut_ws)
         return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    // When the Stage1 kernel gives each (sequence, kv-head part) one wave anyway, that wave
-    // runs the whole sequence as one split: the same attention (up to rounding), without
-    // writing and re-reading num_kv_splits rows per head (with sinks too: the sink enters
-    // split 0, the only split then).  Stage2's merge of one split is the identity, so the
-    // Stage1 kernel writes the output rows and LSE itself (mid_o is not written then).
     Stage1Args a{q_rot_ws, kv_cache, block_table, seq_lens, pair_lut_ws, mid_o, B, Hq, Hk, D,
                  block_size, max_blocks_per_seq, cache_block_stride, num_kv_splits, layout,
                  attn_scale, sinks};
     a.query_dtype = query_dtype;
-    if (check_stage1(a) == TQ4_OK && auto_xdl_waves(a) == 1) {
+    const int waves = check_stage1(a) == TQ4_OK ? decode_waves(a) : 0;
+    if (waves > 0) {
         if (!out || !lse || !query || !rot_t)
             return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
         if (out_dtype != TQ4_F32 && out_dtype != TQ4_BF16 && out_dtype != TQ4_F16)
             return fail(TQ4_E_INVALID, "tq4_full_decode: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
-        a.S = 1;
         a.out = out;
         a.out_dtype = out_dtype;
         a.lse = lse;
-        if (rot_applies(a) && aligned(query, 16)) {
+        if (waves == 1 && rot_applies(a) && aligned(query, 16)) {
             // one launch: the workgroup of each sequence rotates its query into LDS (the
             // workspaces q_rot_ws and pair_lut_ws are not written)
             a.query = query;
@@ -620,7 +647,7 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
             return run_stage1(a, TQ4_KERNEL_XDL, st);
         }
         const int rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
-        return rc ? rc : run_stage1(a, TQ4_KERNEL_XDL, st);
+        return rc ? rc : run_parts(a, waves, st);
     }
     // one launch rotates the query and writes the pair LUT
     int rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
@@ -660,8 +687,8 @@ int tq4_full_decode_noalloc(const void *query, int query_dtype, const float *rot
     rc = check_stage1(a);  // invalid arguments report their own error, not a workspace size
     if (rc)
         return rc;
-    const bool one_split = auto_xdl_waves(a) == 1;
-    const size_t mid_bytes = one_split ? 0 : (size_t)B * Hq * num_kv_splits * (D + 1) * sizeof(float);
+    const bool one_wave = decode_waves(a) == 1;  // the step then writes no part rows
+    const size_t mid_bytes = one_wave ? 0 : (size_t)B * Hq * num_kv_splits * (D + 1) * sizeof(float);
     const size_t need = lut_bytes + q_bytes + mid_bytes;
     if (need > kScratchBytes)
         return fail(TQ4_E_INVALID,
