@@ -128,6 +128,21 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
                     float attn_scale, const float *sinks, tq4_stream_t stream);
 
 /*
+ * The full decode step of the other presets: key_bits / value_bits 8/4 (FP8 keys: the query
+ * is used unrotated; rot_t, centroids and q_rot_ws may be NULL; where the 16x16x32 kernel does
+ * not apply the query must be TQ4_F32), 3/4 and 3/3 (centroids [8]).  query must be 16-byte
+ * aligned.  Workspaces and outputs as in tq4_full_decode.
+ * Replaces: triton_turboquant_decode_attention reference/soa_decode_v1.py:485-643 with
+ *           key_fp8 / mse_bits = 3.
+ */
+int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_t, const float *centroids,
+                           const uint8_t *kv_cache, const int32_t *block_table, const int32_t *seq_lens,
+                           float *q_rot_ws, float *mid_o, void *out, int out_dtype, float *lse, int B, int Hq,
+                           int Hk, int D, int block_size, int max_blocks_per_seq, int64_t cache_block_stride,
+                           int num_kv_splits, int layout, float attn_scale, const float *sinks, int key_bits,
+                           int value_bits, tq4_stream_t stream);
+
+/*
  * tq4_full_decode without caller workspaces: the pair LUT, the rotated queries and the
  * Stage1 rows live in a 40 MiB device array the library holds on every GPU it runs on (from
  * its load until the process ends), so the call allocates nothing -- no hipMalloc, no

@@ -13,7 +13,8 @@ import torch
 from conftest import to_dev
 from oracle import native
 from oracle import stage1 as ostage
-from tq4_decode import ops, workloads
+from tq4_decode import aos_decode, codebook, ops, soa_decode, workloads
+from tq4_decode.layout import slot_bytes_fp8, slot_bytes_preset
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +82,63 @@ def test_sinks_enter_the_first_part_only(dev):
                                          num_kv_heads=8, sinks=sinks), w.seq_lens)
     assert np.abs(out.cpu().numpy() - ro).max() <= 1e-4
     assert np.abs(lse.cpu().numpy() - rl).max() <= 1e-4
+
+
+def _preset_cache(dev, rng, bits, blocks, bs, hk, layout):
+    """A cache written by the writer from random keys and values (every block full)."""
+    kb, vb = bits
+    slot = slot_bytes_fp8(128) if kb == 8 else slot_bytes_preset(128, kb, vb)
+    cache = torch.zeros(blocks, bs, hk, slot, dtype=torch.uint8, device=dev)
+    n = blocks * bs
+    k, v = (to_dev(rng.standard_normal((n, hk, 128)).astype(np.float32), dev).bfloat16() for _ in range(2))
+    slots = torch.arange(n, dtype=torch.int32, device=dev)
+    if kb == 8:
+        return ops.store_fp8(k, v, cache, slots, layout=layout), None
+    cents = to_dev(codebook.centroids(128, kb), dev)
+    rot = to_dev(workloads.random_orthogonal(rng, 128), dev)
+    ops.store_preset(k, v, cache, slots, rot, to_dev(codebook.midpoints(128, kb), dev), cents, key_bits=kb,
+                     value_bits=vb, layout=layout, norm_correction=layout == "soa")
+    return cache, cents
+
+
+# (block size 8 runs on the VALU kernel: rotation or conversion, Stage1 and Stage2 as before)
+@pytest.mark.parametrize("layout,hk,group,bs,lens", [
+    ("soa", 8, 4, 16, EDGES), ("aos", 8, 4, 16, EDGES), ("soa", 4, 8, 32, EDGES), ("aos", 4, 6, 16, EDGES),
+    ("soa", 2, 16, 16, [700] * 5), ("soa", 8, 4, 8, EDGES[:6]), ("soa", 8, 4, 16, [40] * 300)])
+@pytest.mark.parametrize("bits", [(8, 4), (3, 4), (3, 3)])
+@pytest.mark.parametrize("view", ["contiguous", "strided", "off by 2 bytes"])
+def test_preset_step_matches_the_separate_launches(dev, bits, layout, hk, group, bs, lens, view):
+    """Outputs in fp16 against Stage1 over 16 splits + Stage2: both merge fp32 sums, so they differ
+    by 1e-5 before the last rounding and by one fp16 unit (2^-10) after it."""
+    if view == "off by 2 bytes" and bits != (8, 4):
+        pytest.skip("the rotation takes 16-byte aligned queries")
+    rng = np.random.default_rng(940 + bits[0] + hk)
+    batch, hq = len(lens), hk * group
+    need = [max(1, -(-n // bs)) for n in lens]
+    cache, cents = _preset_cache(dev, rng, bits, sum(need), bs, hk, layout)
+    table = np.zeros((batch, max(need)), np.int32)
+    perm = rng.permutation(sum(need))
+    for b, n in enumerate(need):
+        table[b, :n] = perm[sum(need[:b]):sum(need[:b]) + n]
+    bt, sl = to_dev(table, dev), to_dev(np.asarray(lens, np.int32), dev)
+    x = to_dev(rng.standard_normal(batch * hq * 128 * 2 + 1).astype(np.float32), dev).half()
+    if view == "strided":
+        query = x[1:].view(batch, hq, 256)[:, :, ::2]
+    else:
+        query = x[1 if "off" in view else 0:][:batch * hq * 128].view(batch, hq, 128)
+    pit = to_dev(workloads.random_orthogonal(rng, 128), dev)
+    entry = (soa_decode if layout == "soa" else aos_decode).triton_turboquant_decode_attention
+    got = entry(query, cache, bt, sl, pit.t().contiguous(), cents, 128 ** -0.5, bits[0],
+                128 if bits[0] == 8 else 16 * bits[0] + 2, bits[1], key_fp8=bits[0] == 8, norm_correction=True,
+                PiT=pit, max_num_kv_splits=16)
+    if bits[0] == 8:
+        mid = ops.stage1_fp8(query.float().contiguous(), cache, bt, sl, num_kv_splits=16, layout=layout)
+    else:
+        mid = ops.stage1_preset(ops.rotate_query(query.contiguous(), pit), cache, bt, sl, cents, key_bits=bits[0],
+                                value_bits=bits[1], num_kv_splits=16, layout=layout)
+    ref, _ = ops.stage2(mid, sl)
+    torch.cuda.synchronize()
+    a, r = got.float().cpu().numpy(), ref.cpu().numpy()
+    live = np.asarray(lens) > 0
+    assert np.isnan(a[~live]).all()
+    assert np.all(np.abs(a[live] - r[live]) <= 1e-5 + 2.0 ** -10 * np.abs(r[live]))

@@ -709,6 +709,20 @@ __device__ __forceinline__ void load_q_rows(float4 (&qx)[8], const float *__rest
         qx[m] = *reinterpret_cast<const float4 *>(qr + d);
     }
 }
+// FP8 keys in the full decode step: the same dims of an unrotated bf16 / fp16 query row (exact
+// in fp32), read as the caller has it -- a conversion launch over B x Hq rows would cost ~4 us.
+template <typename T>
+__device__ __forceinline__ void load_query_rows_fp8(float4 (&qx)[8], const T *__restrict__ query, int64_t head_row,
+                                                    int g) {
+    typedef T t8 __attribute__((ext_vector_type(8)));
+    const T *qr = query + head_row * kHeadDim + 16 * g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const t8 v = *reinterpret_cast<const t8 *>(qr + 64 * (i >> 1) + 8 * (i & 1));
+        qx[2 * i] = float4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+        qx[2 * i + 1] = float4{(float)v[4], (float)v[5], (float)v[6], (float)v[7]};
+    }
+}
 // A q row whose largest |q * scale| reaches 2^15 is first scaled by the power of two 2^e
 // (e < 0) that puts it in [2^14, 2^15), inside the f16 range of the hi part; the returned
 // 2^-e (1 for every other row, so their scores are unchanged bit for bit) multiplies the
@@ -1359,7 +1373,8 @@ __device__ __forceinline__ void rot_column_tile(const half8 (&ah)[G / 2][4], con
 // ROT (with PARTS; 1: bf16 queries, 2: fp16): a workgroup is the nvh waves of one sequence
 // (grid (B)), which rotate the query themselves (q_rot is not read: `query`, `rot_t`, and
 // pair_lut holds the 16 centroids).
-// KF8: the FP8-key preset (K one E4M3 byte per dim, no norm, the query not rotated).
+// KF8: the FP8-key preset (K one E4M3 byte per dim, no norm, the query not rotated; with PARTS
+// q_rot holds the query's own q_dtype rows).
 // KB3: the 3-bit-key / 4-bit-value preset (pair_lut then holds the 8 centroids).
 template <int LAYOUT, int G, int WPE, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false, int ROT = 0>
 __global__ __launch_bounds__(ROT ? kWave * kRotGroupWaves : kWave) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
@@ -1370,7 +1385,7 @@ void stage1_xdl_kernel(
     void *__restrict__ out, int out_dtype, float *__restrict__ lse,
     int num_q_heads, int num_kv_heads, int block_size_log2, int max_blocks, int64_t block_stride,
     int slot_pos, int slot_head, int num_splits, float score_scale_log2,
-    const void *__restrict__ query, const float *__restrict__ rot_t) {
+    const void *__restrict__ query, const float *__restrict__ rot_t, int q_dtype) {
     static_assert(G == 4 || G == 8, "4 or 8 q-heads per wave");
     static_assert(ROT == 0 || (PARTS && !KF8 && !KB3), "the query rotation runs in the one-wave 4-bit kernel");
     using QueryT = std::conditional_t<ROT == 1, __bf16, _Float16>;
@@ -1792,7 +1807,13 @@ void stage1_xdl_kernel(
                                  num_q_heads, lane & 15, lane >> 4);
         rot_load_cols(rot_cols, rot_t, threadIdx.x / kWave, lane & 15, lane >> 4);
     } else {
-        load_q_rows(q_rows, q_rot, (int64_t)b * num_q_heads + hb + hl, lane >> 4, KF8);
+        const int64_t head_row = (int64_t)b * num_q_heads + hb + hl;
+        if (KF8 && PARTS && q_dtype == kOutBf16)
+            load_query_rows_fp8(q_rows, reinterpret_cast<const __bf16 *>(q_rot), head_row, lane >> 4);
+        else if (KF8 && PARTS && q_dtype == kOutF16)
+            load_query_rows_fp8(q_rows, reinterpret_cast<const _Float16 *>(q_rot), head_row, lane >> 4);
+        else
+            load_q_rows(q_rows, q_rot, head_row, lane >> 4, KF8);
     }
     chunk_addresses(blk0);
     issue_slots(0, min(64, total) - 1, 0, FIRST_SLOTS);

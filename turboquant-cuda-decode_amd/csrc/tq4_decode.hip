@@ -266,7 +266,7 @@ template <int LAYOUT, int G> void launch_xdl(const Stage1Args &a, hipStream_t st
                                 : &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, true, false, false, false, 2>;
         launch(kernel, dim3(a.B), dim3(tq4::kWave * nvh), st, a.q_rot, a.cache, a.bt, a.seq_lens, a.lut,
                a.mid_o, a.sinks, a.out, a.out_dtype, a.lse, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks,
-               a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, a.query, a.rot_t);
+               a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, a.query, a.rot_t, a.query_dtype);
         return;
     }
     const dim3 grid(nvh, a.out ? xdl_waves_of<LAYOUT, G, true>(a) : xdl_waves_of<LAYOUT, G, false>(a), a.B);
@@ -279,7 +279,7 @@ template <int LAYOUT, int G> void launch_xdl(const Stage1Args &a, hipStream_t st
         kernel = a.out ? xdl_kernel<LAYOUT, G, true, false, true>() : xdl_kernel<LAYOUT, G, false, false, true>();
     launch(kernel, grid, dim3(tq4::kWave), st, a.q_rot, a.cache, a.bt, a.seq_lens, a.lut,
            a.mid_o, a.sinks, a.out, a.out_dtype, a.lse, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks,
-           a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, nullptr, nullptr);
+           a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, nullptr, nullptr, a.query_dtype);
 }
 
 template <int LAYOUT> int dispatch_simple(const Stage1Args &a, hipStream_t st) {
@@ -653,6 +653,53 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
     int rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
     if (rc)
         return rc;
+    rc = run_stage1(a, TQ4_KERNEL_AUTO, st);
+    if (rc)
+        return rc;
+    return tq4_stage2(mid_o, seq_lens, out, out_dtype, lse, B, Hq, D, a.S, stream);
+}
+
+int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_t, const float *centroids,
+                           const uint8_t *kv_cache, const int32_t *block_table, const int32_t *seq_lens,
+                           float *q_rot_ws, float *mid_o, void *out, int out_dtype, float *lse, int B, int Hq,
+                           int Hk, int D, int block_size, int max_blocks_per_seq, int64_t cache_block_stride,
+                           int num_kv_splits, int layout, float attn_scale, const float *sinks, int key_bits,
+                           int value_bits, tq4_stream_t stream) {
+    const bool fp8 = key_bits == 8 && value_bits == 4;
+    if (!fp8 && (key_bits == 4 || !preset_supported(key_bits, value_bits)))
+        return fail(TQ4_E_UNSUPPORTED, "tq4_full_decode_preset: key_bits / value_bits %d / %d unsupported "
+                                       "(8/4, 3/4, 3/3)", key_bits, value_bits);
+    if (!query || !out || !lse || (!fp8 && (!rot_t || !centroids)))
+        return fail(TQ4_E_INVALID, "tq4_full_decode_preset: null pointer argument");
+    if (query_dtype != TQ4_F32 && query_dtype != TQ4_BF16 && query_dtype != TQ4_F16)
+        return fail(TQ4_E_INVALID, "tq4_full_decode_preset: query_dtype must be 0, 1 or 2");
+    if (out_dtype != TQ4_F32 && out_dtype != TQ4_BF16 && out_dtype != TQ4_F16)
+        return fail(TQ4_E_INVALID, "tq4_full_decode_preset: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    Stage1Args a{fp8 ? static_cast<const float *>(query) : q_rot_ws, kv_cache, block_table, seq_lens, centroids,
+                 mid_o, B, Hq, Hk, D, block_size, max_blocks_per_seq, cache_block_stride, num_kv_splits, layout,
+                 attn_scale, sinks};
+    a.key_fp8 = fp8;
+    a.key_bits = fp8 ? 0 : key_bits;
+    a.value_bits = value_bits;
+    a.query_dtype = query_dtype;
+    int rc = check_stage1(a);
+    if (rc)
+        return rc;
+    const int waves = decode_waves(a);
+    if (fp8 && waves == 0 && query_dtype != TQ4_F32)
+        return fail(TQ4_E_UNSUPPORTED, "tq4_full_decode_preset: FP8 keys on the VALU kernel take an fp32 query");
+    if (!fp8) {
+        rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, nullptr, nullptr, st);
+        if (rc)
+            return rc;
+    }
+    if (waves > 0) {
+        a.out = out;
+        a.out_dtype = out_dtype;
+        a.lse = lse;
+        return run_parts(a, waves, st);
+    }
     rc = run_stage1(a, TQ4_KERNEL_AUTO, st);
     if (rc)
         return rc;

@@ -409,6 +409,41 @@ def full_decode(query, rotation_t, kv_cache, block_table, seq_lens, centroids, n
     return ws.out, ws.lse
 
 
+def _full_decode_preset(query, rotation_t, kv_cache, block_table, seq_lens, centroids, ws, *, key_bits,
+                        value_bits, layout, attn_scale, sinks):
+    """The full step of the FP8-key (``key_bits`` 8) and 3-bit presets into ``ws.out`` / ``ws.lse``."""
+    fp8 = key_bits == 8
+    for t, n in ((block_table, "block_table"), (seq_lens, "seq_lens")):
+        _check_tensor(t, n, torch.int32)
+    _require(query.is_cuda and query.dtype in DTYPES, "invalid query")
+    B, Hq, D = query.shape
+    slot = slot_bytes_fp8(D) if fp8 else slot_bytes_preset(D, key_bits, value_bits)
+    bs, Hk, stride, lid = _cache_geometry(kv_cache, slot, layout, " (FP8 keys)" if fp8 else "")
+    _require(Hq % Hk == 0, "Hq must be a multiple of Hk")
+    _require(block_table.dim() == 2 and block_table.size(0) == B, "block_table batch mismatch")
+    _require(seq_lens.dim() == 1 and seq_lens.size(0) == B, "seq_lens batch mismatch")
+    tensors = [query, kv_cache, block_table, seq_lens, ws.mid_o, ws.out, ws.lse]
+    if not fp8:
+        _check_tensor(rotation_t, "rotation_t", torch.float32)
+        _require(tuple(rotation_t.shape) == (D, D), f"requires D={HEAD_DIM}")
+        _require(centroids.numel() == 1 << key_bits, f"{key_bits}-bit keys need {1 << key_bits} centroids")
+        tensors += [rotation_t, centroids]
+    _require(len({t.device for t in tensors}) == 1, "all tensors must be on the same device")
+    mfma = bs >= 16 and bs & (bs - 1) == 0 and stride % 16 == 0
+    if fp8 and not (mfma and query.data_ptr() % 16 == 0):
+        # the VALU kernel takes fp32 rows, and both take them aligned
+        query = ws.q_rot.copy_(query)
+    rc = _lib.load().tq4_full_decode_preset(
+        query.data_ptr(), DTYPES[query.dtype], None if fp8 else rotation_t.data_ptr(),
+        None if fp8 else centroids.data_ptr(), kv_cache.data_ptr(), block_table.data_ptr(), seq_lens.data_ptr(),
+        ws.q_rot.data_ptr(), ws.mid_o.data_ptr(), ws.out.data_ptr(), DTYPES[ws.out.dtype], ws.lse.data_ptr(),
+        B, Hq, Hk, D, bs, block_table.size(1), stride, ws.mid_o.size(2), lid,
+        1.0 / math.sqrt(D) if attn_scale is None else float(attn_scale), _check_sinks(sinks, Hq, query.device),
+        key_bits, value_bits, _stream(query.device))
+    _lib.check(rc, "tq4_full_decode_preset")
+    return ws.out
+
+
 def _buffer_view(buf, shape, dtype):
     """``buf`` cut to ``shape`` (leading sub-block) when it fits and stays contiguous."""
     if buf is None or buf.dtype != dtype or buf.dim() != len(shape):
@@ -477,12 +512,9 @@ def turboquant_decode_attention(query, kv_cache, block_table, seq_lens, Pi, cent
     if key_fp8:
         _require(value_quant_bits == 4, "FP8 keys are built with 4-bit values")
         _require(key_packed_size == HEAD_DIM, f"key_packed_size must be {HEAD_DIM} for FP8 keys")
-        # the unrotated query (reference/soa_decode_v1.py:528-534), as fp32
-        ws.q_rot.copy_(query)
-        stage1_fp8(ws.q_rot, kv_cache, block_table, seq_lens, ws.mid_o, layout=layout,
-                   attn_scale=scale, sinks=sinks)
-        stage2(ws.mid_o, seq_lens, ws.out, ws.lse)
-        return ws.out
+        # the unrotated query (reference/soa_decode_v1.py:528-534)
+        return _full_decode_preset(query.contiguous(), None, kv_cache, block_table, seq_lens, None, ws, key_bits=8,
+                                   value_bits=4, layout=layout, attn_scale=scale, sinks=sinks)
     _require((mse_bits, value_quant_bits) in PRESETS,
              f"MSE key / value bits must be one of {PRESETS}")
     want = HEAD_DIM * mse_bits // 8 + 2
@@ -493,13 +525,9 @@ def turboquant_decode_attention(query, kv_cache, block_table, seq_lens, Pi, cent
         PiT = Pi.t().contiguous()
     query = query.contiguous()
     if mse_bits != 4 or value_quant_bits != 4:
-        # 3-bit-key presets: rotation, Stage1 over the preset cache, Stage2
-        rotate_query(query, PiT, ws.q_rot)
-        stage1_preset(ws.q_rot, kv_cache, block_table, seq_lens, centroids.float().contiguous(),
-                      ws.mid_o, key_bits=mse_bits, value_bits=value_quant_bits, layout=layout,
-                      attn_scale=scale, sinks=sinks)
-        stage2(ws.mid_o, seq_lens, ws.out, ws.lse)
-        return ws.out
+        return _full_decode_preset(query, PiT, kv_cache, block_table, seq_lens, centroids.float().contiguous(), ws,
+                                   key_bits=mse_bits, value_bits=value_quant_bits, layout=layout, attn_scale=scale,
+                                   sinks=sinks)
     out, _ = full_decode(query, PiT, kv_cache, block_table, seq_lens, centroids, S,
                          layout=layout, out_dtype=query.dtype, attn_scale=scale, workspace=ws,
                          sinks=sinks)
