@@ -107,15 +107,14 @@ int tq4_build_pair_lut(const float *centroids, float *pair_lut, int n_centroids,
                        tq4_stream_t stream);
 
 /*
- * Full decode step: rotate query into q_rot_ws, build the pair LUT into
- * pair_lut_ws (512 floats), Stage1 into mid_o, merge into out / lse; sinks as in
- * tq4_stage1_ex (may be NULL).  q_rot_ws, pair_lut_ws and mid_o (B*Hq*num_kv_splits*(D+1)
- * floats) are workspaces, their contents after the call unspecified: on the 16x16x32 kernel
- * mid_o holds one row per Stage1 wave (at most num_kv_splits per sequence and head) in a
- * layout of its own instead of one per split.  When every (sequence, kv-head) gets one wave,
- * Stage1 writes out / lse itself (mid_o unwritten), and for TQ4_BF16 / TQ4_F16 queries with
- * Hk * (waves per kv-head) dividing 8 the same launch also rotates the query (q_rot_ws and
- * pair_lut_ws unwritten).
+ * Full decode step: query rotation, attention over the cache, output rows and LSE; sinks as in
+ * tq4_stage1_ex (may be NULL).  query must be 16-byte aligned.  q_rot_ws (B*Hq*D floats),
+ * pair_lut_ws (512 floats) and mid_o (B*Hq*num_kv_splits*(D+1) floats) are workspaces, their
+ * contents after the call unspecified.  Where the 16x16x32 kernel applies, one launch rotates
+ * the query (TQ4_F32 queries: a launch before it, into q_rot_ws) and runs the attention: with
+ * one workgroup per sequence it writes out / lse itself, else it leaves at most num_kv_splits
+ * rows per sequence and head in mid_o, in a layout of its own, for a merge launch.  Other
+ * shapes: rotation and pair LUT, Stage1, Stage2.
  * Replaces: tq4_cuda_v7_full cuda/tq4_cuda_v7.cu:78-84 plus the q rotation of
  *           triton_turboquant_decode_attention reference/soa_decode_v1.py:485-643.
  */
@@ -147,7 +146,7 @@ int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_
  * Stage1 rows live in a 40 MiB device array the library holds on every GPU it runs on (from
  * its load until the process ends), so the call allocates nothing -- no hipMalloc, no
  * allocator.  Shapes whose workspace exceeds the array (2 KiB LUT + B*Hq*D*4 bytes of
- * q_rot + B*Hq*S*(D+1)*4 bytes of Stage1 rows unless every sequence gets one wave) are
+ * q_rot + B*Hq*S*(D+1)*4 bytes of rows, these only while B * (head parts) <= half the waves the device holds) are
  * rejected with TQ4_E_INVALID.  Calls that overlap on one GPU share the array and race:
  * serialize them (one stream, or events).  Otherwise as tq4_full_decode.
  * No counterpart in the reference: for callers that cannot allocate (code under graph

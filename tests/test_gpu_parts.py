@@ -1,11 +1,13 @@
-"""The full decode step's part rows: a sequence's 16-token tiles divided among its Stage1 waves,
-one row per wave, merged by ``merge_parts_kernel``.
+"""The full decode step as one kernel plus (where a sequence has several workgroups) the merge:
+the list of all sequences' 16-token tiles cut into equal stretches, one row per workgroup and
+head.
 
-Sizes are where the division, the part count and the block-table guess can go wrong: lengths
-around tile edges, fewer tiles than waves, as many parts as split rows (no count mark), more
-parts than the merge reads at once, batches past the ranked deal's 64 sequences, blocks of
-several tiles with full and partly used tables.  Bar, against the float64 / C oracle: 1e-4 on
-outputs and LSE (fp32 outputs; the Stage1 requirement)."""
+Sizes are where the cut, the waves' runs, the part count and the block-table guess can go
+wrong: lengths around tile edges, fewer tiles than waves, as many parts as rows (no count mark)
+and more than the merge reads at once, stretches over several sequences and sequences over
+several stretches, batches past 64 sequences and past the device, one to eight head parts per
+workgroup, blocks of several tiles with full and partly used tables.  Bar, against the float64 /
+C oracle: 1e-4 on outputs and LSE (fp32 outputs; the Stage1 requirement)."""
 import numpy as np
 import pytest
 import torch
@@ -33,6 +35,16 @@ CASES = {
     "equal, odd, blocks of 64": ([2041] * 64, 32, 8, 4, 64, "soa"),
     "equal, one tile": ([7] * 9, 32, 8, 4, 32, "soa"),
     "all empty": ([0] * 5, 32, 8, 4, 16, "soa"),
+    "one long sequence": ([20011], 32, 8, 4, 16, "soa"),
+    "one long sequence, one row": ([3001], 1, 8, 4, 16, "soa"),
+    "long and short": ([9000, 1, 40, 0, 700], 8, 4, 8, 16, "aos"),
+    "three kv-heads": ([1500, 700, 1, 0, 90, 333], 32, 3, 4, 16, "soa"),
+    "five kv-heads, group of 6": ([1500, 700, 1, 0, 90, 333], 32, 5, 6, 16, "aos"),
+    "eight waves of one head part": ([4000, 3000], 16, 1, 8, 32, "soa"),
+    "130 equal sequences": ([1000] * 130, 16, 8, 4, 16, "soa"),
+    "130 ragged sequences": (list(np.random.default_rng(6).integers(0, 900, 130)), 16, 8, 4, 16, "soa"),
+    "300 ragged sequences": (list(np.random.default_rng(7).integers(0, 600, 300)), 8, 8, 8, 16, "soa"),
+    "one token each, 200 sequences, wide table": ([1] * 199 + [2000], 16, 8, 4, 16, "soa"),
     "ragged, 150 sequences": (list(np.random.default_rng(5).integers(0, 700, 150)), 32, 2, 4, 16, "soa"),
 }
 

@@ -152,21 +152,6 @@ __device__ __forceinline__ void build_key_table(uint32_t *tbl, const LutRows &v,
     }
 }
 
-// The rows i = w (mod nw) of the table (entries lane + 64 i), for a table that nw waves of a
-// workgroup build together.
-template <int LAYOUT>
-__device__ __forceinline__ void build_key_table_rows(uint32_t *tbl, const LutRows &v, int lane, int w, int nw) {
-#pragma unroll
-    for (int i = 0; i < 256 / kWave; ++i) {
-        if (i % nw != w)
-            continue;
-        const int e = lane + kWave * i;
-        const uint32_t p_lo = split_f16(v.r[i].x), p_hi = split_f16(v.r[i].y);
-        tbl[2 * e] = (p_lo & 0xFFFFu) | (p_hi << 16);
-        tbl[2 * e + 1] = (p_lo >> 16) | (p_hi & 0xFFFF0000u);
-    }
-}
-
 // 3-bit keys: entry e = a | b << 3 holds ((c_hi[a], c_hi[b]), (c_lo[a], c_lo[b])) -- the
 // codes of a dim pair are 6 consecutive bits; one entry per lane (centroids [8]).
 __device__ __forceinline__ void build_key_table3(uint32_t *tbl, const float *centroids, int lane) {
@@ -514,30 +499,24 @@ struct Deal {
     int len;         // seq_lens[b], as the deal read it
 };
 
-// The units dealt and the estimated stream positions of a sequence of len tokens (sequence
-// bb, 0 past the batch).  PARTS: the units are its 16-token tiles, one position each; else its
-// live splits, each with its tiles (one more when it straddles a tile edge), as the stream
-// pads them.
+// Live splits and estimated stream positions of a sequence of len tokens (sequence bb, 0
+// past the batch): each split's tiles (one more when it straddles a tile edge), as the
+// stream pads them.
 struct SeqLoad {
     int live;
     uint32_t est;
     int len;
-    int per;  // estimated positions per unit
+    int per;  // estimated positions per split
 };
-template <bool PARTS> __device__ __forceinline__ SeqLoad sequence_load_len(int len, int S) {
+__device__ __forceinline__ SeqLoad sequence_load_len(int len, int S) {
     len = max(len, 0);
-    if constexpr (PARTS) {
-        const int tiles = (len + 15) >> 4;
-        return SeqLoad{tiles, (uint32_t)tiles, len, 1};
-    }
     const int split_len = div_pos(len + S - 1, S);
     const int live = split_len > 0 ? (len + split_len - 1) / split_len : 0;
     const int per = ((split_len + 15) >> 4) + 1;
     return SeqLoad{live, (uint32_t)live * (uint32_t)per, len, per};
 }
-template <bool PARTS>
 __device__ __forceinline__ SeqLoad sequence_load(const int32_t *__restrict__ seq_lens, int B, int S, int bb) {
-    return sequence_load_len<PARTS>(bb < B ? seq_lens[bb] : 0, S);
+    return sequence_load_len(bb < B ? seq_lens[bb] : 0, S);
 }
 
 // Inclusive prefix sum over the wave's 64 lanes: shifts within each 16-lane row, then the
@@ -576,8 +555,8 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 // by bisection on its load (lane-wide counts of the waves at least that heavy), then by its
 // place among the waves of exactly that load.  Any x -> p bijection keeps the deal exact.
 // lane_len: seq_lens[lane] (0 past the batch), read by the caller.
-template <bool PARTS> __device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane) {
-    const SeqLoad q = sequence_load_len<PARTS>(lane_len, S);
+__device__ Deal deal_ranked(int lane_len, int B, int S, int nw, int x, int lane) {
+    const SeqLoad q = sequence_load_len(lane_len, S);
     const uint32_t est_total = wave_sum(q.est);
     const int n_live = __builtin_popcountll(__ballot(q.live > 0));
     // spare waves before prefix pre: floor(pre * spare / total) with one fp32 ratio -- monotone
@@ -585,10 +564,10 @@ template <bool PARTS> __device__ Deal deal_ranked(int lane_len, int B, int S, in
     const float ratio = est_total > 0 ? (float)((int64_t)nw * B - n_live) / (float)est_total : 0.f;
     auto cut = [&](uint32_t pre) { return (int)floorf((float)pre * ratio); };
     const uint32_t est_out = wave_scan(q.est);
-    const int k = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), PARTS ? min(q.live, S) : q.live) : 0;
-    const int per = q.live > 0 ? q.per : 0;  // positions per unit
-    // live / k and live % k: an fp32 quotient is within 1 of it for live below 2^22 (live <= S;
-    // PARTS: 2^22 tiles are 2^26 tokens), so one correction step makes it exact
+    const int k = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), q.live) : 0;
+    const int per = q.live > 0 ? q.per : 0;  // positions per split
+    // live / k and live % k: an fp32 quotient is within 1 of it for live below 2^22 (live <= S),
+    // so one correction step makes it exact
     int qd = 0, r = 0;
     if (k > 0) {
         qd = (int)((float)q.live * __builtin_amdgcn_rcpf((float)k));
@@ -630,7 +609,6 @@ template <bool PARTS> __device__ Deal deal_ranked(int lane_len, int B, int S, in
     return Deal{sq, j, __builtin_amdgcn_readlane(k, sq), __builtin_amdgcn_readlane(q.len, sq)};
 }
 
-template <bool PARTS>
 __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, int nw, int x, int lane) {
     // equal lengths: every sequence keeps its nw waves, as the deal would give them
     const int len0 = seq_lens[0];
@@ -646,12 +624,12 @@ __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, i
     if (equal)
         return Deal{x / nw, x % nw, nw, len0};
     if (B <= kWave)
-        return deal_ranked<PARTS>(lane_len, B, S, nw, x, lane);
-    const SeqLoad first = sequence_load_len<PARTS>(lane_len, S);
+        return deal_ranked(lane_len, B, S, nw, x, lane);
+    const SeqLoad first = sequence_load_len(lane_len, S);
     uint32_t est_total = 0;
     int n_live = 0;
     for (int c0 = 0; c0 < B; c0 += kWave) {
-        const SeqLoad q = c0 == 0 ? first : sequence_load<PARTS>(seq_lens, B, S, c0 + lane);
+        const SeqLoad q = c0 == 0 ? first : sequence_load(seq_lens, B, S, c0 + lane);
         est_total += (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(q.est), kWave - 1);
         n_live += __builtin_popcountll(__ballot(q.live > 0));
     }
@@ -662,10 +640,9 @@ __device__ Deal deal_waves(const int32_t *__restrict__ seq_lens, int B, int S, i
     uint32_t est_carry = 0;
     int wave_carry = 0;
     for (int c0 = 0; c0 < B; c0 += kWave) {
-        const SeqLoad q = c0 == 0 ? first : sequence_load<PARTS>(seq_lens, B, S, c0 + lane);
+        const SeqLoad q = c0 == 0 ? first : sequence_load(seq_lens, B, S, c0 + lane);
         const uint32_t est_out = est_carry + wave_scan(q.est);
-        const int mine =
-            q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), PARTS ? min(q.live, S) : q.live) : 0;
+        const int mine = q.live > 0 ? min(1 + cut(est_out) - cut(est_out - q.est), q.live) : 0;
         const int w_out = wave_carry + (int)wave_scan((uint32_t)mine);
         const int w_in = w_out - mine;
         const uint64_t hit = __ballot(x >= w_in && x < w_out);
@@ -707,20 +684,6 @@ __device__ __forceinline__ void load_q_rows(float4 (&qx)[8], const float *__rest
     for (int m = 0; m < 8; ++m) {
         const int d = kf8 ? (m < 4 ? 16 * g + 4 * m : 64 + 16 * g + 4 * (m - 4)) : 32 * g + 4 * m;
         qx[m] = *reinterpret_cast<const float4 *>(qr + d);
-    }
-}
-// FP8 keys in the full decode step: the same dims of an unrotated bf16 / fp16 query row (exact
-// in fp32), read as the caller has it -- a conversion launch over B x Hq rows would cost ~4 us.
-template <typename T>
-__device__ __forceinline__ void load_query_rows_fp8(float4 (&qx)[8], const T *__restrict__ query, int64_t head_row,
-                                                    int g) {
-    typedef T t8 __attribute__((ext_vector_type(8)));
-    const T *qr = query + head_row * kHeadDim + 16 * g;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const t8 v = *reinterpret_cast<const t8 *>(qr + 64 * (i >> 1) + 8 * (i & 1));
-        qx[2 * i] = float4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-        qx[2 * i + 1] = float4{(float)v[4], (float)v[5], (float)v[6], (float)v[7]};
     }
 }
 // A q row whose largest |q * scale| reaches 2^15 is first scaled by the power of two 2^e
@@ -1157,62 +1120,6 @@ __device__ __forceinline__ void stash_split(const State &st, const floatx4 (&acc
         img[lc.n * Cap::head_floats + j * (kHeadDim + 1) + kHeadDim] = lse_of(st.negm, safe_l);
 }
 
-// Output element conversion of the fused epilogue (the same roundings as Stage2's).
-__device__ __forceinline__ void put_out(void *out, int dtype, int64_t i, float v) {
-    if (dtype == kOutBf16)
-        static_cast<__bf16 *>(out)[i] = (__bf16)v;
-    else if (dtype == kOutF16)
-        static_cast<_Float16 *>(out)[i] = (_Float16)v;
-    else
-        static_cast<float *>(out)[i] = v;
-}
-
-// One split per sequence: with a single live split Stage2's merge is the identity (weight
-// exp(0) = 1, sum 1), so the wave writes the final output rows and LSE itself -- the same
-// values Stage2 would write, without the mid_o round trip.
-// Heads nh .. G-1 of the wave are padding (a GQA group that is not a multiple of G).
-template <int G, bool V3>
-__device__ __forceinline__ void emit_output(const State &st, const floatx4 (&acc)[8], const LaneConst &lc,
-                                            void *out, int out_dtype, float *lse, int64_t row0, int nh) {
-    int h0;
-    float o[G / 4][8], safe_l;
-    finish_rows<G, V3>(st, acc, lc, h0, o, safe_l);
-    const int64_t r = (row0 + h0) * kHeadDim + 8 * lc.n;
-#pragma unroll
-    for (int k = 0; k < G / 4; ++k)
-        if (h0 + k < nh)
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                put_out(out, out_dtype, r + k * kHeadDim + i, o[k][i]);
-    if (lc.g == 0 && lc.n < nh)
-        lse[row0 + lc.n] = lse_of(st.negm, safe_l);
-}
-
-// Row `wid` of each head's part rows: the wave's outputs and LSE, and, from the sequence's
-// first wave, how many rows there are (layout: part_rows / part_lse in stage2.h).
-template <int G, bool V3>
-__device__ __forceinline__ void emit_part(const State &st, const floatx4 (&acc)[8], const LaneConst &lc,
-                                          float *__restrict__ parts, int64_t total_rows, int64_t row0, int num_splits,
-                                          int wid, int run_waves, int nh) {
-    int h0;
-    float o[G / 4][8], safe_l;
-    finish_rows<G, V3>(st, acc, lc, h0, o, safe_l);
-    typedef float float4a __attribute__((ext_vector_type(4), aligned(4)));
-#pragma unroll
-    for (int k = 0; k < G / 4; ++k)
-        if (h0 + k < nh) {
-            float *r = part_row(parts, row0 + h0 + k, num_splits, wid) + 8 * lc.n;
-            *reinterpret_cast<float4a *>(r) = float4a{o[k][0], o[k][1], o[k][2], o[k][3]};
-            *reinterpret_cast<float4a *>(r + 4) = float4a{o[k][4], o[k][5], o[k][6], o[k][7]};
-        }
-    if (lc.g == 0 && lc.n < nh) {
-        float *l = part_lse(parts, total_rows, row0 + lc.n, num_splits);
-        l[wid] = part_lse_value(lse_of(st.negm, safe_l));
-        if (wid == 0 && run_waves < num_splits)
-            l[num_splits - 1] = part_count_mark(run_waves);
-    }
-}
-
 // Write image slots 0 .. ns-1 to the rows of splits s0 .. s0+ns-1 (heads 0 .. nh-1; the
 // rest are padding).  Rows of one head and consecutive splits are consecutive in mid_o
 // [B, Hq, S, D + 1], so head h's slots are one run of ns * 129 floats.  One wave: its LDS
@@ -1245,107 +1152,6 @@ __device__ __forceinline__ void flush_splits(const float *img, float *__restrict
     asm volatile("" ::: "memory");
 }
 
-// ---- Query rotation inside the one-split kernel (ROT) --------------------------------
-// A workgroup holds the nvh waves of one sequence (nvh = its kv-heads times the parts of
-// their GQA groups, a divisor of 8: at most two waves per SIMD of one CU).  Together they
-// compute the sequence's rotated queries q_rot = query @ rot_t into LDS with the operands
-// and the MFMA order of rotate_mfma_kernel, so the rows are bit-identical to that launch's:
-// each query row scaled by the power of two that puts its largest |x| in [2^14, 2^15) (exact
-// in f16 for fp16 / bf16 queries), rot_t as f16 hi + lo parts, D[rows 4g .. 4g+3][col n] of
-// output column tile c per row tile.  Wave w takes the column tiles c = w, w + nvh, ..., so it
-// reads 8 KB of rot_t per tile (one column slab), not the whole 64 KB.
-constexpr int kRotGroupWaves = 8;
-constexpr int kQRowFloats = kHeadDim + 4;  // LDS row of a rotated query (rows 16 bytes apart in bank)
-
-// Query elements of the lane for every row tile of the sequence: row 16t + n (rows past Hq
-// repeat the last one and are not stored), elements 32kb + 8g .. +7 -- the A operand of
-// rotate_mfma_kernel.  Hq <= 8 G, so G / 2 row tiles.
-template <int G> struct RotRows {
-    uint4 raw[G / 2][4];
-};
-template <typename InT, int G>
-__device__ __forceinline__ void rot_load_rows(RotRows<G> &a, const InT *__restrict__ query, int64_t row_base,
-                                              int hq, int n, int g) {
-#pragma unroll
-    for (int t = 0; t < G / 2; ++t) {
-        const int row = min(16 * t + n, hq - 1);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-            a.raw[t][kb] = *reinterpret_cast<const uint4 *>(query + (row_base + row) * kHeadDim + 32 * kb + 8 * g);
-    }
-}
-// rot_t[32kb + 8g + j][16c + n]: the lane's B operand of column tile c (fp32, split later).
-struct RotCols {
-    float v[4][8];
-};
-__device__ __forceinline__ void rot_load_cols(RotCols &b, const float *__restrict__ rot_t, int c, int n, int g) {
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            b.v[kb][j] = rot_t[(32 * kb + 8 * g + j) * kHeadDim + 16 * c + n];
-}
-// Scaled f16 A operands of every row tile and the scale exponents of the D rows each lane
-// receives (row 4g + i of tile t).
-template <typename InT, int G>
-__device__ __forceinline__ void rot_a_operands(const RotRows<G> &a, half8 (&ah)[G / 2][4], int (&e_out)[G / 2][4],
-                                               int g) {
-    typedef InT in8 __attribute__((ext_vector_type(8)));
-#pragma unroll
-    for (int t = 0; t < G / 2; ++t) {
-        float amax = 0.f;
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            const in8 p = __builtin_bit_cast(in8, a.raw[t][kb]);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                amax = fmaxf(amax, fabsf(to_float<InT>(p[j])));
-        }
-        amax = rot_row_max(amax);
-        const int e = (amax > 0.f && amax < __builtin_inff()) ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            e_out[t][i] = __shfl(e, 4 * g + i, kWave);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            const in8 p = __builtin_bit_cast(in8, a.raw[t][kb]);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                ah[t][kb][j] = (_Float16)__builtin_ldexpf(to_float<InT>(p[j]), e);
-        }
-    }
-}
-// Column tile c of every row tile into the LDS rows qbuf [Hq][kQRowFloats].
-template <int G>
-__device__ __forceinline__ void rot_column_tile(const half8 (&ah)[G / 2][4], const int (&e_out)[G / 2][4],
-                                                const RotCols &b, float *qbuf, int c, int hq, int n, int g) {
-    half8 bh[4], bl[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            bh[kb][j] = (_Float16)b.v[kb][j];
-            bl[kb][j] = (_Float16)(b.v[kb][j] - (float)bh[kb][j]);
-        }
-#pragma unroll
-    for (int t = 0; t < G / 2; ++t) {
-        if (16 * t >= hq)
-            break;
-        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            acc = mfma(ah[t][kb], bh[kb], acc);
-            acc = mfma(ah[t][kb], bl[kb], acc);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 16 * t + 4 * g + i;
-            if (row < hq)
-                qbuf[row * kQRowFloats + 16 * c + n] = __builtin_ldexpf(acc[i], -e_out[t][i]);
-        }
-    }
-}
-
 // One wave handles a run of consecutive live splits of one (sequence, kv-head).  Their
 // tiles form one stream: split s contributes its n_s tiles padded to an even count, the
 // wave's last split as many more as make the stream whole ring turns (padding positions
@@ -1360,35 +1166,17 @@ __device__ __forceinline__ void rot_column_tile(const half8 (&ah)[G / 2][4], con
 // nh .. G-1 as padding (zero queries, never written).  Grid x runs over the (part, kv-head)
 // pairs, vh = part * Hk + kv-head.
 //
-// PARTS (the full decode step, whose split rows nobody else reads): no splits.  A sequence's
-// 16-token tiles are divided among its waves, each wave takes one contiguous run of them and
-// leaves one row per head (mid_o in the layout of part_row, stage2.h; merged by
-// merge_parts_kernel).  Against num_splits rows this drops the mid_o traffic of all but one
-// row per wave, the split ends inside the stream, and, for lengths that are not a multiple of
-// 16 num_splits, the tiles that two splits share and the padding of each split.  With one
-// wave per (sequence, kv-head part) (gridDim.y = 1) that wave owns the whole sequence and
-// writes the final output rows (out, out_dtype) and LSE itself.
-// Measured, full step with 32 splits, B64 x 32/8 heads: 4096 tokens 82.6 -> 68.8 us (AoS 97.1 ->
-// 84.2), ragged 512..8192 95.3 -> 77.3.
-// ROT (with PARTS; 1: bf16 queries, 2: fp16): a workgroup is the nvh waves of one sequence
-// (grid (B)), which rotate the query themselves (q_rot is not read: `query`, `rot_t`, and
-// pair_lut holds the 16 centroids).
-// KF8: the FP8-key preset (K one E4M3 byte per dim, no norm, the query not rotated; with PARTS
-// q_rot holds the query's own q_dtype rows).
+// KF8: the FP8-key preset (K one E4M3 byte per dim, no norm, the query not rotated).
 // KB3: the 3-bit-key / 4-bit-value preset (pair_lut then holds the 8 centroids).
-template <int LAYOUT, int G, int WPE, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false, int ROT = 0>
-__global__ __launch_bounds__(ROT ? kWave * kRotGroupWaves : kWave) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <int LAYOUT, int G, int WPE, bool KF8 = false, bool KB3 = false, bool V3 = false>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void stage1_xdl_kernel(
     const float *__restrict__ q_rot, const uint8_t *__restrict__ cache,
     const int32_t *__restrict__ block_table, const int32_t *__restrict__ seq_lens,
     const float *__restrict__ pair_lut, float *__restrict__ mid_o, const float *__restrict__ sinks,
-    void *__restrict__ out, int out_dtype, float *__restrict__ lse,
     int num_q_heads, int num_kv_heads, int block_size_log2, int max_blocks, int64_t block_stride,
-    int slot_pos, int slot_head, int num_splits, float score_scale_log2,
-    const void *__restrict__ query, const float *__restrict__ rot_t, int q_dtype) {
+    int slot_pos, int slot_head, int num_splits, float score_scale_log2) {
     static_assert(G == 4 || G == 8, "4 or 8 q-heads per wave");
-    static_assert(ROT == 0 || (PARTS && !KF8 && !KB3), "the query rotation runs in the one-wave 4-bit kernel");
-    using QueryT = std::conditional_t<ROT == 1, __bf16, _Float16>;
     constexpr int TPL = G / 4;
     constexpr int RING = 4;
     // ring slots of the first chunk issued before the K table and q operands are built (the
@@ -1396,21 +1184,9 @@ void stage1_xdl_kernel(
     // queue behind fewer of the other waves' loads
     constexpr int FIRST_SLOTS = 2;
     const int block_size = 1 << block_size_log2;
-    int vh, wid, b;
-    if constexpr (ROT) {
-        // wave w of the sequence's workgroup; with 8 waves (2 per SIMD: waves w and w + 4 share
-        // one) SIMD s gets parts 2s and 2s + 1, one even and one odd kv-head (see below)
-        const int w = threadIdx.x / kWave;
-        vh = blockDim.x == kWave * 8 ? 2 * (w & 3) + (w >> 2) : w;
-        wid = 0;
-        b = blockIdx.x;
-    } else {
-        vh = blockIdx.x;
-        wid = blockIdx.y;
-        b = blockIdx.z;
-    }
-    const int nw = ROT ? 1 : gridDim.y;
-    if constexpr (!ROT && (LAYOUT == 1 || KF8 || KB3)) {
+    int vh = blockIdx.x, wid = blockIdx.y, b = blockIdx.z;
+    const int nw = gridDim.y;
+    if constexpr (LAYOUT == 1 || KF8 || KB3) {
         // Workgroups are dealt to the XCDs round-robin by linear id (8 on gfx950), so with
         // the plain map kv-head h runs on XCD h.  An AoS slot (or a preset's SoA record of
         // 192, 112 or 96 bytes) of kv-head h shares 128-byte lines with those of h - 1 and h + 1: the kv-heads of one (sequence, wave)
@@ -1434,9 +1210,9 @@ void stage1_xdl_kernel(
     // ones would end last: the second half of the grid takes kv-head h ^ 1 instead, and
     // every SIMD runs one even and one odd kv-head.  The kv-heads of one (sequence, wave)
     // pair still start together (and share an XCD where the map above puts them on one).
-    if (!ROT && (gridDim.x & 1) == 0 && 2 * (wid + nw * b) >= nw * (int)gridDim.z)
+    if ((gridDim.x & 1) == 0 && 2 * (wid + nw * b) >= nw * (int)gridDim.z)
         vh ^= 1;
-    const int lane = threadIdx.x % kWave;
+    const int lane = threadIdx.x;
     const int group = num_q_heads / num_kv_heads;
     const int kvh = vh % num_kv_heads, part = vh / num_kv_heads;
     const int hb = kvh * group + part * G;       // the wave's first q-head
@@ -1447,16 +1223,8 @@ void stage1_xdl_kernel(
     // lengths make right.  When the first chunk's entries turn out to be exactly these, the
     // registers serve it and the block-table read leaves the path to the first KV loads;
     // otherwise the guess has warmed L2 for the real reads.
-    const int guess_b = b;
-    int guess_block, guess_tile = 0;  // lane i: the block of the guessed run's tile i (PARTS: from guess_tile)
-    if constexpr (PARTS) {
-        const int tl = block_size_log2 - 4, most = max_blocks << tl, q = most / nw;
-        guess_tile = wid * q + min(wid, most - q * nw);
-        guess_block = min((guess_tile + lane) >> tl, max_blocks - 1);
-    } else {
-        guess_block = min(wid * ((max_blocks + nw - 1) / nw) + lane, max_blocks - 1);
-    }
-    const int bt_guess = block_table[(int64_t)b * max_blocks + guess_block];
+    const int guess_b = b, guess_first = wid * ((max_blocks + nw - 1) / nw);
+    const int bt_guess = block_table[(int64_t)b * max_blocks + min(guess_first + lane, max_blocks - 1)];
     // The pair-LUT rows do not depend on the sequence: they go out first; the K table and the
     // q operands are built once the first tiles' loads are on their way.
     static_assert(!(KF8 && KB3), "one key format");
@@ -1467,58 +1235,26 @@ void stage1_xdl_kernel(
     constexpr bool STG8 = KF8 && LAYOUT == 0;
     using RK = std::conditional_t<STG8, RawRec3, std::conditional_t<KF8, RawK8, std::conditional_t<STG, RawRec, std::conditional_t<KB3, RawK3, RawK<LAYOUT>>>>>;
     LutRows lut_rows{};
-    if constexpr (ROT) {
-        // from the centroids themselves: entry e = (c[e & 15], c[e >> 4]), the pair-LUT row
-#pragma unroll
-        for (int i = 0; i < 256 / kWave; ++i) {
-            const int e = lane + kWave * i;
-            lut_rows.r[i] = float2{pair_lut[e & 15], pair_lut[e >> 4]};
-        }
-    } else if constexpr (!KF8 && !KB3) {
+    if constexpr (!KF8 && !KB3)
         lut_rows = load_lut_rows(pair_lut, lane);
-    }
     // the head's sink logit (a dummy read when there are none: one unconditional load here
     // keeps the waits before the first KV loads from covering it)
     const float sink = *(sinks ? sinks + hb + hl : q_rot);
-    int run_waves = nw;  // waves sharing this wave's sequence and kv-head
-    int dealt_len = 0;
-    const bool whole = PARTS && nw == 1;  // the wave owns its sequence (of this kv-head part)
-    if (ROT || whole) {
-        dealt_len = seq_lens[b];
-    } else {
-        const Deal d = deal_waves<PARTS>(seq_lens, gridDim.z, num_splits, nw, wid + nw * b, lane);
-        if (d.b < 0)
-            return;
-        b = d.b;
-        wid = d.wid;
-        run_waves = d.nw;
-        dealt_len = d.len;
-        if (PARTS)  // equal lengths: every sequence is dealt nw waves, at most one per tile
-            run_waves = min(run_waves, (max(dealt_len, 0) + 15) >> 4);
-    }
-    const int seq_len = dealt_len;
-    // split partition: L = ceil(len / S); live splits are those with s * L < len.  PARTS: the
-    // "splits" are the 16-token tiles, of which the wave's run makes one row
-    const int split_len = PARTS ? 16 : div_pos(max(seq_len, 0) + num_splits - 1, num_splits);
-    const int live = PARTS ? (max(seq_len, 0) + 15) >> 4
-                           : split_len > 0 ? min(num_splits, div_pos(seq_len + split_len - 1, split_len)) : 0;
+    const Deal d = deal_waves(seq_lens, gridDim.z, num_splits, nw, wid + nw * b, lane);
+    if (d.b < 0)
+        return;
+    b = d.b;
+    wid = d.wid;
+    const int run_waves = d.nw;  // waves sharing this wave's sequence and kv-head
+    const int seq_len = d.len;
+    // split partition: L = ceil(len / S); live splits are those with s * L < len
+    const int split_len = div_pos(max(seq_len, 0) + num_splits - 1, num_splits);
+    const int live = split_len > 0 ? min(num_splits, div_pos(seq_len + split_len - 1, split_len)) : 0;
     // run x of the W runs of this (sequence, kv-head): live splits from x q + min(x, r), q + 1 of
     // them for x < r and q after (q = live / W, r = live % W)
-    const int run_q = PARTS && run_waves <= 0 ? 0 : div_pos(live, run_waves), run_r = live - run_q * run_waves;
+    const int run_q = div_pos(live, run_waves), run_r = live - run_q * run_waves;
     const int s_lo = wid * run_q + min(wid, run_r);
-    const int s_hi = wid < run_waves ? s_lo + run_q + (wid < run_r ? 1 : 0) : s_lo;
-    if constexpr (PARTS) {
-        if (whole && live == 0) {
-            // an empty sequence: what Stage2 writes for it (0 / 0 and ln 0); with ROT every
-            // wave of the workgroup returns here (one sequence), before its barrier
-            const int64_t r0 = ((int64_t)b * num_q_heads + hb) * kHeadDim;
-            for (int i = lane; i < nh * kHeadDim; i += kWave)
-                put_out(out, out_dtype, r0 + i, __builtin_nanf(""));
-            if (lane < nh)
-                lse[(int64_t)b * num_q_heads + hb + lane] = -__builtin_inff();
-            return;
-        }
-    }
+    const int s_hi = s_lo + run_q + (wid < run_r ? 1 : 0);
     if (s_lo >= s_hi)
         return;
 
@@ -1537,11 +1273,10 @@ void stage1_xdl_kernel(
     constexpr int kRec = record_bytes<LAYOUT, KF8, KB3, V3>();
     constexpr int kStage = STG ? 16 * kRec + 16 : STG8 ? 16 * kRec : 0;
     __shared__ __align__(16) uint8_t recbuf[kStage > 0 ? kStage : 16];
-    // split starts of a chunk, one byte per stream position (chunk_tiles; PARTS has no splits)
-    __shared__ uint8_t marks[PARTS ? 1 : kWave];
-    using Cap = SpanCap<LAYOUT, G, WPE, (KF8 ? 0 : KTable<LAYOUT>::words * 4) + kStage + (PARTS ? 0 : kWave)>;
-    __shared__ __align__(16) float img[PARTS ? 4 : Cap::floats];  // PARTS: rows go out from registers
-    __shared__ __align__(16) float qbuf[ROT ? kRotGroupWaves * G * kQRowFloats : 4];
+    // split starts of a chunk, one byte per stream position (chunk_tiles)
+    __shared__ uint8_t marks[kWave];
+    using Cap = SpanCap<LAYOUT, G, WPE, (KF8 ? 0 : KTable<LAYOUT>::words * 4) + kStage + kWave>;
+    __shared__ __align__(16) float img[Cap::floats];
     half8 bq[8];
     float q_unscale = 1.f;  // 2^-e of the lane's q row (q_operands)
 
@@ -1573,9 +1308,7 @@ void stage1_xdl_kernel(
     int sp_tf = 0, sp_nt = 0, sp_base = 0;
     int e_log2 = -1;  // log2 of the positions of every split of the run when they are one power of two
     int total = 0;
-    if constexpr (PARTS) {
-        total = n_run;
-    } else if (run_in_lanes) {
+    if (run_in_lanes) {
         const int st0 = (s_lo + min(lane, n_run - 1)) * split_len, en = min(st0 + split_len, seq_len);
         sp_tf = st0 >> 4;
         sp_nt = ((en - 1) >> 4) - sp_tf + 1;
@@ -1604,8 +1337,8 @@ void stage1_xdl_kernel(
     int cur = s_lo;
     int img_s0 = s_lo;  // split of image slot 0
     int cur_start = cur * split_len;
-    int cur_end = min(PARTS ? 16 * s_hi : cur_start + split_len, seq_len);
-    int cur_stop = PARTS ? 0 : split_stop(cur);
+    int cur_end = min(cur_start + split_len, seq_len);
+    int cur_stop = split_stop(cur);
 
     // Lane i of base_lo / base_hi holds the address of the 16-token piece at stream
     // position j0 + i of the current chunk (its KV block plus the piece's offset), lane i
@@ -1718,11 +1451,7 @@ void stage1_xdl_kernel(
     // Lane i: the tile and mask of stream position j0 + i and the block-table entry of that
     // tile (read here; the addresses come from chunk_addresses).
     auto chunk_tiles = [&](int j0, int nchunk) {
-        if constexpr (PARTS) {
-            const int p = j0 + min(lane, nchunk - 1);
-            tile_lane = s_lo + min(p, n_run - 1);
-            mask_lane = p < n_run ? tile_lane : -(1 << 24);  // padding: no valid token
-        } else if (run_in_lanes && e_log2 >= 0) {
+        if (run_in_lanes && e_log2 >= 0) {
             // every split takes 2^e_log2 positions (the tail's go to the last one)
             const int p = j0 + min(lane, nchunk - 1);
             const int i = min(p >> e_log2, n_run - 1);
@@ -1767,13 +1496,8 @@ void stage1_xdl_kernel(
             }
         }
         const int bidx = (16 * tile_lane) >> block_size_log2;
-        if constexpr (PARTS) {
-            // the run starts where the guess did: lane i of the guess holds tile i's block
-            if (j0 == 0 && b == guess_b && s_lo == guess_tile)
-                return __shfl(bt_guess, tile_lane - s_lo, kWave);
-            return bt[bidx];
-        }
-        const bool guessed = j0 == 0 && b == guess_b && __ballot(bidx != guess_block) == 0;
+        const bool guessed = j0 == 0 && b == guess_b &&
+                             __ballot(bidx != min(guess_first + lane, max_blocks - 1)) == 0;
         return guessed ? bt_guess : bt[bidx];
     };
     auto chunk_addresses = [&](int blk) {
@@ -1794,62 +1518,22 @@ void stage1_xdl_kernel(
     };
 
     // The first chunk's first loads go out before the K table and the q operands are built,
-    // and the q (or rotation) loads between its block-table read and those: loads complete in
+    // and the q loads between its block-table read and those: loads complete in
     // issue order, so the first KV addresses wait for the block table alone and the q rows
     // arrive under the first KV loads.
     const int blk0 = chunk_tiles(0, min(64, total));
     float4 q_rows[8];
-    RotRows<G> rot_rows;
-    RotCols rot_cols;
-    const int nvh = ROT ? (int)(blockDim.x / kWave) : 1;
-    if constexpr (ROT) {
-        rot_load_rows<QueryT, G>(rot_rows, static_cast<const QueryT *>(query), (int64_t)b * num_q_heads,
-                                 num_q_heads, lane & 15, lane >> 4);
-        rot_load_cols(rot_cols, rot_t, threadIdx.x / kWave, lane & 15, lane >> 4);
-    } else {
-        const int64_t head_row = (int64_t)b * num_q_heads + hb + hl;
-        if (KF8 && PARTS && q_dtype == kOutBf16)
-            load_query_rows_fp8(q_rows, reinterpret_cast<const __bf16 *>(q_rot), head_row, lane >> 4);
-        else if (KF8 && PARTS && q_dtype == kOutF16)
-            load_query_rows_fp8(q_rows, reinterpret_cast<const _Float16 *>(q_rot), head_row, lane >> 4);
-        else
-            load_q_rows(q_rows, q_rot, head_row, lane >> 4, KF8);
-    }
+    load_q_rows(q_rows, q_rot, (int64_t)b * num_q_heads + hb + hl, lane >> 4, KF8);
     chunk_addresses(blk0);
     issue_slots(0, min(64, total) - 1, 0, FIRST_SLOTS);
-    if constexpr (ROT) {
-        // the sequence's rotated queries into qbuf (column tiles w, w + nvh, ... of this wave)
-        half8 ah[G / 2][4];
-        int e_out[G / 2][4];
-        rot_a_operands<QueryT, G>(rot_rows, ah, e_out, lc.g);
-        const int w = threadIdx.x / kWave;
-        rot_column_tile<G>(ah, e_out, rot_cols, qbuf, w, num_q_heads, lc.n, lc.g);
-        for (int c = w + nvh; c < kHeadDim / 16; c += nvh) {
-            rot_load_cols(rot_cols, rot_t, c, lc.n, lc.g);
-            rot_column_tile<G>(ah, e_out, rot_cols, qbuf, c, num_q_heads, lc.n, lc.g);
-        }
-        // the shared K table: wave w builds rows i = w (mod nvh) of it
-        build_key_table_rows<LAYOUT>(ktab, lut_rows, lane, w, nvh);
-        // LDS writes done, then the workgroup barrier (the KV loads stay in flight: no
-        // vmcnt wait, unlike __syncthreads)
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (hl != ((lane & 15) & (G - 1)))  // padding head: a zero query
 #pragma unroll
         for (int m = 0; m < 8; ++m)
-            q_rows[m] = *reinterpret_cast<const float4 *>(qbuf + (hb + hl) * kQRowFloats + 32 * lc.g + 4 * m);
-        if (hl != ((lane & 15) & (G - 1)))
-#pragma unroll
-            for (int m = 0; m < 8; ++m)
-                q_rows[m] = float4{0.f, 0.f, 0.f, 0.f};
-    } else {
-        if (hl != ((lane & 15) & (G - 1)))  // padding head: a zero query
-#pragma unroll
-            for (int m = 0; m < 8; ++m)
-                q_rows[m] = float4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (KB3)
-            build_key_table3(ktab, pair_lut, lane);
-        else if constexpr (!KF8)
-            build_key_table<LAYOUT>(ktab, lut_rows, lane);
-    }
+            q_rows[m] = float4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (KB3)
+        build_key_table3(ktab, pair_lut, lane);
+    else if constexpr (!KF8)
+        build_key_table<LAYOUT>(ktab, lut_rows, lane);
     q_unscale = q_operands(bq, q_rows, lc.n, score_scale_log2);
     issue_slots(0, min(64, total) - 1, FIRST_SLOTS, RING);
     // one wave: its LDS writes complete before its later LDS reads; only the compiler must
@@ -1896,9 +1580,8 @@ void stage1_xdl_kernel(
                 if (k & 1) {
                     issue_vpos(vr[k - 1], pos[(k + 3) % RING], moff_lane, min(j + k - 1 + RING, last));
                     issue_vpos(vr[k], pos[k % RING], moff_lane, min(j + k + RING, last));
-                    // a split ends after an odd stage (PARTS: the one row ends with the
-                    // stream and is written after the loop)
-                    if (!PARTS && j + k + 1 == pos_base + cur_stop) {
+                    // a split ends after an odd stage
+                    if (j + k + 1 == pos_base + cur_stop) {
                         stash_split<G, Cap, V3>(st, acc, lc, img, cur - img_s0);
                         if (cur + 1 == s_hi || cur + 1 - img_s0 == Cap::splits) {
                             flush_splits<G, Cap>(img, mid_o, row0, num_splits, img_s0, cur + 1 - img_s0, lane, nh);
@@ -1919,13 +1602,6 @@ void stage1_xdl_kernel(
             }
             j += RING;
         } while (j <= last);
-    }
-    if constexpr (PARTS) {
-        if (ROT || whole)
-            emit_output<G, V3>(st, acc, lc, out, out_dtype, lse, row0, nh);
-        else
-            emit_part<G, V3>(st, acc, lc, mid_o, (int64_t)gridDim.z * num_q_heads, row0, num_splits, wid, run_waves,
-                             nh);
     }
 }
 

@@ -18,6 +18,7 @@
 #include "stage1_simple.h"
 #include "stage1_xdl.h"
 #include "stage2.h"
+#include "step.h"
 #include "store.h"
 
 namespace {
@@ -31,15 +32,19 @@ thread_local hipEvent_t g_time_start = nullptr, g_time_stop = nullptr;
 // Every kernel launch goes through here: arguments are converted to the kernel's
 // parameter types (the event-stamping launch passes them by address).
 template <typename... KArgs, typename... Args>
-void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t st, Args... args) {
+void launch_lds(void (*kernel)(KArgs...), dim3 grid, dim3 block, int lds_bytes, hipStream_t st, Args... args) {
     static_assert(sizeof...(KArgs) == sizeof...(Args), "argument count");
     if (g_time_start || g_time_stop) {
         const hipEvent_t a = g_time_start, b = g_time_stop;
         g_time_start = g_time_stop = nullptr;
-        hipExtLaunchKernelGGL(kernel, grid, block, 0, st, a, b, 0, static_cast<KArgs>(args)...);
+        hipExtLaunchKernelGGL(kernel, grid, block, lds_bytes, st, a, b, 0, static_cast<KArgs>(args)...);
     } else {
-        hipLaunchKernelGGL(kernel, grid, block, 0, st, static_cast<KArgs>(args)...);
+        hipLaunchKernelGGL(kernel, grid, block, lds_bytes, st, static_cast<KArgs>(args)...);
     }
+}
+template <typename... KArgs, typename... Args>
+void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t st, Args... args) {
+    launch_lds(kernel, grid, block, 0, st, args...);
 }
 
 int fail(int code, const char *fmt, ...) {
@@ -83,20 +88,10 @@ struct Stage1Args {
     int S, layout;  // TQ4_LAYOUT_*
     float scale;
     const float *sinks = nullptr;  // [Hq] sink logits of split 0, or null
-    // set: a full decode step on the XDL kernel (PARTS): part rows in mid_o, or with one wave
-    // per (sequence, kv-head part) the final rows
-    void *out = nullptr;
-    int out_dtype = TQ4_F32;
-    float *lse = nullptr;
     bool key_fp8 = false;  // the FP8-key preset (VALU kernel; pair LUT unused)
     // > 0: the key_bits / value_bits preset on the VALU kernel; lut holds the 2^key_bits
     // centroids (not the pair LUT)
     int key_bits = 0, value_bits = 4;
-    // set (with out): the one-split kernel rotates this query itself (TQ4_BF16 / TQ4_F16 rows
-    // [B, Hq, D]) with rot_t, and lut holds the 16 centroids instead of the pair LUT
-    const void *query = nullptr;
-    int query_dtype = TQ4_F32;
-    const float *rot_t = nullptr;
     // filled by check_stage1: kernel layout (0 SoA, 1 AoS) and the AoS slot strides
     int kl = 0, slot_pos = 0, slot_head = 0;
 };
@@ -194,7 +189,7 @@ int xdl_parts(const Stage1Args &a) {
 // whole rounds of the waves the GPU holds at the kernel's occupancy.  `slots` caches that
 // count per kernel instance (computed on the first call; concurrent first calls compute the
 // same value).  TQ4_STAGE1_WAVES overrides W (a tuning knob; results do not depend on it).
-int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int> &slots, int per_simd) {
+int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int> &slots) {
     static const int forced = [] {
         const char *e = getenv("TQ4_STAGE1_WAVES");
         return e ? atoi(e) : 0;
@@ -208,7 +203,7 @@ int waves_per_sequence(const Stage1Args &a, const void *kernel, std::atomic<int>
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tq4::kWave, 0) == hipSuccess &&
             cus > 0 && per_cu > 0)
-            held = cus * std::min(per_cu, 4 * per_simd);
+            held = cus * per_cu;
         else
             held = 256 * 4 * 2;
         slots.store(held, std::memory_order_relaxed);
@@ -231,55 +226,24 @@ template <int LAYOUT, int G> constexpr int xdl_waves_per_simd() {
     return LAYOUT == 0 && G == 4 ? TQ4_XDL_WAVES_PER_SIMD : 2;
 }
 
-// The kernel of one key / value format; PARTS: the full decode step's form of it.
-template <int LAYOUT, int G, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false> constexpr auto xdl_kernel() {
-    return &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, xdl_waves_per_simd<LAYOUT, G>(), PARTS, KF8, KB3, V3>;
-}
-template <int LAYOUT, int G, bool PARTS, bool KF8 = false, bool KB3 = false, bool V3 = false>
-int xdl_waves(const Stage1Args &a) {
+template <int LAYOUT, int G, bool KF8 = false, bool KB3 = false, bool V3 = false>
+void launch_xdl_format(const Stage1Args &a, hipStream_t st) {
     static std::atomic<int> slots{0};
-    return waves_per_sequence(a, reinterpret_cast<const void *>(xdl_kernel<LAYOUT, G, PARTS, KF8, KB3, V3>()), slots,
-                              xdl_waves_per_simd<LAYOUT, G>());
+    const auto kernel = &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, xdl_waves_per_simd<LAYOUT, G>(), KF8, KB3, V3>;
+    const int waves = waves_per_sequence(a, reinterpret_cast<const void *>(kernel), slots);
+    launch(kernel, dim3(a.Hk * xdl_parts(a), waves, a.B), dim3(tq4::kWave), st, a.q_rot, a.cache, a.bt, a.seq_lens,
+           a.lut, a.mid_o, a.sinks, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks, a.stride, a.slot_pos, a.slot_head, a.S,
+           a.scale * tq4::kLog2e);
 }
-template <int LAYOUT, int G, bool PARTS> int xdl_waves_of(const Stage1Args &a) {
-    if (a.key_fp8)
-        return xdl_waves<LAYOUT, G, PARTS, true>(a);
-    if (a.key_bits == 3)
-        return a.value_bits == 3 ? xdl_waves<LAYOUT, G, PARTS, false, true, true>(a)
-                                 : xdl_waves<LAYOUT, G, PARTS, false, true>(a);
-    return xdl_waves<LAYOUT, G, PARTS>(a);
-}
-
-// The one-split kernel that rotates the query itself: one workgroup per sequence holding its
-// Hk * parts waves, which must divide 8 (two waves per SIMD of one CU).
-bool rot_applies(const Stage1Args &a) {
-    const int nvh = a.Hk * xdl_parts(a);
-    return (a.query_dtype == TQ4_BF16 || a.query_dtype == TQ4_F16) && 8 % nvh == 0;
-}
-
 template <int LAYOUT, int G> void launch_xdl(const Stage1Args &a, hipStream_t st) {
-    constexpr int wpe = xdl_waves_per_simd<LAYOUT, G>();
-    const int nvh = a.Hk * xdl_parts(a);
-    if (a.query) {  // one split per sequence, the rotation inside (Stage2 fused)
-        const auto kernel = a.query_dtype == TQ4_BF16
-                                ? &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, true, false, false, false, 1>
-                                : &tq4::xdl::stage1_xdl_kernel<LAYOUT, G, wpe, true, false, false, false, 2>;
-        launch(kernel, dim3(a.B), dim3(tq4::kWave * nvh), st, a.q_rot, a.cache, a.bt, a.seq_lens, a.lut,
-               a.mid_o, a.sinks, a.out, a.out_dtype, a.lse, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks,
-               a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, a.query, a.rot_t, a.query_dtype);
-        return;
-    }
-    const dim3 grid(nvh, a.out ? xdl_waves_of<LAYOUT, G, true>(a) : xdl_waves_of<LAYOUT, G, false>(a), a.B);
-    auto kernel = a.out ? xdl_kernel<LAYOUT, G, true>() : xdl_kernel<LAYOUT, G, false>();
     if (a.key_fp8)
-        kernel = a.out ? xdl_kernel<LAYOUT, G, true, true>() : xdl_kernel<LAYOUT, G, false, true>();
+        launch_xdl_format<LAYOUT, G, true>(a, st);
     else if (a.key_bits == 3 && a.value_bits == 3)
-        kernel = a.out ? xdl_kernel<LAYOUT, G, true, false, true, true>() : xdl_kernel<LAYOUT, G, false, false, true, true>();
+        launch_xdl_format<LAYOUT, G, false, true, true>(a, st);
     else if (a.key_bits == 3)
-        kernel = a.out ? xdl_kernel<LAYOUT, G, true, false, true>() : xdl_kernel<LAYOUT, G, false, false, true>();
-    launch(kernel, grid, dim3(tq4::kWave), st, a.q_rot, a.cache, a.bt, a.seq_lens, a.lut,
-           a.mid_o, a.sinks, a.out, a.out_dtype, a.lse, a.Hq, a.Hk, log2_int(a.bs), a.max_blocks,
-           a.stride, a.slot_pos, a.slot_head, a.S, a.scale * tq4::kLog2e, nullptr, nullptr, a.query_dtype);
+        launch_xdl_format<LAYOUT, G, false, true>(a, st);
+    else
+        launch_xdl_format<LAYOUT, G>(a, st);
 }
 
 template <int LAYOUT> int dispatch_simple(const Stage1Args &a, hipStream_t st) {
@@ -317,17 +281,6 @@ template <int LAYOUT> int dispatch_xdl(const Stage1Args &a, hipStream_t st) {
     return launch_status("stage1_xdl");
 }
 
-// Waves per (sequence, kv-head part) of the full decode step (0 when the 16x16x32 kernel does
-// not apply).
-int decode_waves(const Stage1Args &a) {
-    if (!mfma_applies(a))
-        return 0;
-    const bool g4 = xdl_heads(a) == 4;
-    if (a.kl == 0)
-        return g4 ? xdl_waves_of<0, 4, true>(a) : xdl_waves_of<0, 8, true>(a);
-    return g4 ? xdl_waves_of<1, 4, true>(a) : xdl_waves_of<1, 8, true>(a);
-}
-
 int run_stage1(Stage1Args a, int kernel, hipStream_t st) {
     int rc = check_stage1(a);
     if (rc)
@@ -350,31 +303,6 @@ int run_stage1(Stage1Args a, int kernel, hipStream_t st) {
     if (kernel == TQ4_KERNEL_XDL)
         return a.kl == 0 ? dispatch_xdl<0>(a, st) : dispatch_xdl<1>(a, st);
     return fail(TQ4_E_INVALID, "tq4_stage1_ex: unknown kernel id %d", kernel);
-}
-
-// Rows the merge requests ahead of the part count: 8 cover what a ragged batch usually deals
-// a sequence at up to 8 waves each (more are read in further chunks of 8), 32 the rest.
-constexpr int kMergeSmall = 8, kMergeLarge = 32;
-
-// The attention of a full decode step from rotated queries: Stage1 in part rows, then their
-// merge; `waves` = decode_waves(a).  With one wave per (sequence, kv-head part) Stage1 writes
-// the output rows itself.
-int run_parts(const Stage1Args &a, int waves, hipStream_t st) {
-    const int rc = run_stage1(a, TQ4_KERNEL_XDL, st);
-    if (rc || waves == 1)
-        return rc;
-    const bool small = waves <= kMergeSmall;
-    const dim3 grid(a.Hq, a.B), block(tq4::kWave);
-#define TQ4_MERGE_LAUNCH(T)                                                                                     \
-    launch(small ? &tq4::merge_parts_kernel<T, kMergeSmall> : &tq4::merge_parts_kernel<T, kMergeLarge>, grid, block, \
-           st, a.mid_o, a.seq_lens, static_cast<T *>(a.out), a.lse, a.Hq, a.S)
-    switch (a.out_dtype) {
-    case TQ4_F32: TQ4_MERGE_LAUNCH(float); break;
-    case TQ4_BF16: TQ4_MERGE_LAUNCH(__bf16); break;
-    default: TQ4_MERGE_LAUNCH(_Float16); break;
-    }
-#undef TQ4_MERGE_LAUNCH
-    return launch_status("merge_parts");
 }
 
 int rotate_query(const void *query, int query_dtype, const float *rot_t, float *q_rot, int rows,
@@ -405,6 +333,180 @@ int rotate_query(const void *query, int query_dtype, const float *rot_t, float *
         return fail(TQ4_E_INVALID, "tq4_rotate_query: query_dtype must be 0, 1 or 2");
     }
     return launch_status("rotate_query");
+}
+
+// ---- The full decode step on the 16x16x32 kernel (decode_step_kernel, step.h) ------------
+struct StepIo {
+    const void *query;
+    int query_dtype;
+    const float *rot_t;    // null with FP8 keys
+    float *q_rot_ws;
+    const float *centroids;
+    void *out;
+    int out_dtype;
+    float *lse;
+};
+
+// Waves the device holds at once: every kernel of the step is built for two per SIMD.
+int step_waves_held() {
+    static std::atomic<int> held{0};
+    int h = held.load(std::memory_order_relaxed);
+    if (!h) {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            cus = 256;
+        h = cus * tq4::xdl::kStepWaves;
+        held.store(h, std::memory_order_relaxed);
+    }
+    return h;
+}
+
+// How a step is cut into workgroups, from the shapes alone.
+struct StepPlan {
+    int vw, sw;    // head parts per workgroup, waves per head part
+    int nx;        // workgroups along the list of sequences
+    int per_seq;   // of them per sequence when lengths are equal
+    bool whole;    // one workgroup per sequence, which writes the output rows itself
+};
+int floor_pow2(int64_t x, int most) {
+    int p = 1;
+    while (p < most && 2 * p <= x)
+        p *= 2;
+    return p;
+}
+StepPlan step_plan(const Stage1Args &a, bool have_parts) {
+    const int held = step_waves_held(), nvh = a.Hk * xdl_parts(a);
+    const int64_t pairs = (int64_t)nvh * a.B;  // (sequence, head part) pairs
+    const int64_t tiles = ((int64_t)a.max_blocks * a.bs + 15) / 16;  // of the longest sequence the table can hold
+    // eight head parts per workgroup for 4-bit SoA records (whole 128-byte lines), four for the others,
+    // whose neighbouring heads share lines: B64 x 4096 with 32 / 8 heads takes 66.0 (8) / 67.2 us
+    // (4), AoS 88.8 / 80.4, 3-bit B48 58.8 / 57.5; with two 70.3 to 73.6, 86 to 88 and 66.7
+    const int most_vw = a.kl == 0 && !a.key_fp8 && a.key_bits == 0 ? tq4::xdl::kStepWaves : tq4::xdl::kStepWaves / 2;
+    int vw = 1;
+    while (vw < most_vw && nvh % (2 * vw) == 0)
+        vw *= 2;
+    // whole: one wave per pair fills at least 9/10 of every round, so cutting further would only
+    // add the merge launch; or sequences so short that the waves a pair can have leave each at
+    // most kShortTiles tiles, where the merge costs more than an even cut of ragged lengths gives
+    constexpr int kShortTiles = 8;
+    const int64_t rounds = (pairs + held - 1) / held;
+    const bool full = 10 * pairs >= 9 * rounds * held;
+    int sw = full ? 1 : floor_pow2(held / pairs, tq4::xdl::kStepWaves);
+    if (full || !have_parts || (tiles + sw - 1) / sw <= kShortTiles)
+        return StepPlan{std::min(vw, tq4::xdl::kStepWaves / sw), sw, a.B, 1, true};
+    // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
+    // merge (and no more than there are rows); more waves than that cut ragged batches coarser
+    // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
+    // 8192: 78.1 with one, 82.8 with two, 84.4 with four)
+    constexpr int kMostParts = 16;
+    sw = 1;
+    while (sw < tq4::xdl::kStepWaves && held > pairs * sw * std::min(kMostParts, a.S - 1))
+        sw *= 2;
+    vw = std::min(vw, tq4::xdl::kStepWaves / sw);
+    const int64_t useful = a.B * ((tiles + tq4::xdl::kMinWaveTiles * sw - 1) / (tq4::xdl::kMinWaveTiles * sw));
+    const int nx = (int)std::max<int64_t>(1, std::min<int64_t>(held / (vw * sw) / (nvh / vw), useful));
+    return StepPlan{vw, sw, nx, nx / a.B, false};
+}
+
+template <int LAYOUT, int G, bool ROT, bool KF8 = false, bool KB3 = false, bool V3 = false>
+void launch_step(const tq4::xdl::StepArgs &s, const StepPlan &p, int nvh, hipStream_t st) {
+    launch_lds(&tq4::xdl::decode_step_kernel<LAYOUT, G, ROT, KF8, KB3, V3>, dim3(nvh / p.vw, p.nx),
+               dim3(tq4::kWave * p.vw * p.sw), tq4::xdl::step_lds<LAYOUT, G, ROT, KF8, KB3, V3>(p.vw, p.sw), st, s);
+}
+template <int LAYOUT, int G>
+void launch_step_format(const Stage1Args &a, const tq4::xdl::StepArgs &s, const StepPlan &p, int nvh, hipStream_t st) {
+    const bool rot = s.rot_t != nullptr, v3 = a.value_bits == 3;
+    if (a.key_fp8)
+        launch_step<LAYOUT, G, false, true>(s, p, nvh, st);
+    else if (a.key_bits == 3 && v3)
+        rot ? launch_step<LAYOUT, G, true, false, true, true>(s, p, nvh, st)
+            : launch_step<LAYOUT, G, false, false, true, true>(s, p, nvh, st);
+    else if (a.key_bits == 3)
+        rot ? launch_step<LAYOUT, G, true, false, true>(s, p, nvh, st)
+            : launch_step<LAYOUT, G, false, false, true>(s, p, nvh, st);
+    else
+        rot ? launch_step<LAYOUT, G, true>(s, p, nvh, st) : launch_step<LAYOUT, G, false>(s, p, nvh, st);
+}
+
+// Rows merge_parts_kernel requests ahead of the part count: 8 where a sequence has about that
+// many parts when the lengths are equal (more are read in further chunks), else 32.
+constexpr int kMergeSmall = 8, kMergeLarge = 32;
+
+// The step from checked arguments (check_stage1; mfma_applies).  have_parts: a.mid_o has room
+// for the part rows (else one workgroup per sequence, whatever the batch).
+int run_step(const Stage1Args &a, const StepIo &io, bool have_parts, hipStream_t st) {
+    const StepPlan plan = step_plan(a, have_parts && a.S > 1);
+    const int nvh = a.Hk * xdl_parts(a);
+    tq4::xdl::StepArgs s{};
+    s.query = io.query;
+    s.q_dtype = io.query_dtype;
+    if (!a.key_fp8) {
+        if (io.query_dtype == TQ4_F32) {  // the in-kernel rotation takes 16-bit queries
+            const int rc = rotate_query(io.query, io.query_dtype, io.rot_t, io.q_rot_ws, a.B * a.Hq, a.D, nullptr,
+                                        nullptr, st);
+            if (rc)
+                return rc;
+            s.query = io.q_rot_ws;
+        } else {
+            s.rot_t = io.rot_t;
+        }
+    }
+    s.centroids = io.centroids;
+    s.cache = a.cache;
+    s.block_table = a.bt;
+    s.seq_lens = a.seq_lens;
+    s.sinks = a.sinks;
+    s.parts = a.mid_o;
+    s.out = io.out;
+    s.lse = io.lse;
+    s.block_stride = a.stride;
+    s.score_scale_log2 = a.scale * tq4::kLog2e;
+    s.out_dtype = io.out_dtype;
+    s.batch = a.B;
+    s.num_q_heads = a.Hq;
+    s.num_kv_heads = a.Hk;
+    s.block_size_log2 = log2_int(a.bs);
+    s.max_blocks = a.max_blocks;
+    s.slot_pos = a.slot_pos;
+    s.slot_head = a.slot_head;
+    s.num_splits = a.S;
+    s.group = a.Hq / a.Hk;
+    s.n_hp = xdl_parts(a);
+    s.vw = plan.vw;
+    s.sw = plan.sw;
+    s.per_seq = plan.per_seq;
+    s.whole = plan.whole;
+    if (xdl_heads(a) == 4)
+        a.kl == 0 ? launch_step_format<0, 4>(a, s, plan, nvh, st) : launch_step_format<1, 4>(a, s, plan, nvh, st);
+    else
+        a.kl == 0 ? launch_step_format<0, 8>(a, s, plan, nvh, st) : launch_step_format<1, 8>(a, s, plan, nvh, st);
+    int rc = launch_status("decode_step");
+    if (rc || plan.whole)
+        return rc;
+    const bool small = plan.nx <= kMergeSmall * a.B;
+    const dim3 grid(a.Hq, a.B), block(tq4::kWave);
+#define TQ4_MERGE_LAUNCH(T)                                                                                     \
+    launch(small ? &tq4::merge_parts_kernel<T, kMergeSmall> : &tq4::merge_parts_kernel<T, kMergeLarge>, grid, block, \
+           st, a.mid_o, a.seq_lens, static_cast<T *>(io.out), io.lse, a.Hq, a.S)
+    switch (io.out_dtype) {
+    case TQ4_F32: TQ4_MERGE_LAUNCH(float); break;
+    case TQ4_BF16: TQ4_MERGE_LAUNCH(__bf16); break;
+    default: TQ4_MERGE_LAUNCH(_Float16); break;
+    }
+#undef TQ4_MERGE_LAUNCH
+    return launch_status("merge_parts");
+}
+
+// Checks of a full step's own arguments (the rest is check_stage1's).
+int check_step(const char *what, const void *query, int query_dtype, int out_dtype) {
+    if (query_dtype != TQ4_F32 && query_dtype != TQ4_BF16 && query_dtype != TQ4_F16)
+        return fail(TQ4_E_INVALID, "%s: query_dtype must be 0, 1 or 2", what);
+    if (out_dtype != TQ4_F32 && out_dtype != TQ4_BF16 && out_dtype != TQ4_F16)
+        return fail(TQ4_E_INVALID, "%s: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)", what);
+    if (!aligned(query, 16))
+        return fail(TQ4_E_INVALID, "%s: query must be 16-byte aligned", what);
+    return TQ4_OK;
 }
 
 // The writer for KB-bit K indices / VB-bit V codes over `rows` (token, kv-head) rows.
@@ -615,6 +717,42 @@ int tq4_build_pair_lut(const float *centroids, float *pair_lut, int n_centroids,
     return launch_status("pair_lut");
 }
 
+}  // extern "C"
+
+namespace {
+
+// tq4_full_decode; have_parts: mid_o has room for num_kv_splits rows per sequence and head.
+int full_decode(const void *query, int query_dtype, const float *rot_t, const float *centroids,
+                const uint8_t *kv_cache, const int32_t *block_table, const int32_t *seq_lens, float *q_rot_ws,
+                float *pair_lut_ws, float *mid_o, bool have_parts, void *out, int out_dtype, float *lse, int B, int Hq,
+                int Hk, int D, int block_size, int max_blocks_per_seq, int64_t cache_block_stride, int num_kv_splits,
+                int layout, float attn_scale, const float *sinks, hipStream_t st) {
+    Stage1Args a{q_rot_ws, kv_cache, block_table, seq_lens, pair_lut_ws, mid_o, B, Hq, Hk, D,
+                 block_size, max_blocks_per_seq, cache_block_stride, num_kv_splits, layout,
+                 attn_scale, sinks};
+    if (!query || !rot_t || !out || !lse)
+        return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
+    int rc = check_step("tq4_full_decode", query, query_dtype, out_dtype);
+    if (rc == TQ4_OK)
+        rc = check_stage1(a);
+    if (rc)
+        return rc;
+    if (mfma_applies(a))
+        return run_step(a, StepIo{query, query_dtype, rot_t, q_rot_ws, centroids, out, out_dtype, lse}, have_parts, st);
+    // one launch rotates the query and writes the pair LUT
+    rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
+    if (rc)
+        return rc;
+    rc = run_stage1(a, TQ4_KERNEL_AUTO, st);
+    if (rc)
+        return rc;
+    return tq4_stage2(mid_o, seq_lens, out, out_dtype, lse, B, Hq, D, a.S, st);
+}
+
+}  // namespace
+
+extern "C" {
+
 int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
                     const float *centroids, const uint8_t *kv_cache,
                     const int32_t *block_table, const int32_t *seq_lens, float *q_rot_ws,
@@ -624,39 +762,10 @@ int tq4_full_decode(const void *query, int query_dtype, const float *rot_t,
                     float attn_scale, const float *sinks, tq4_stream_t stream) {
     if (!centroids || !pair_lut_ws)
         return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    Stage1Args a{q_rot_ws, kv_cache, block_table, seq_lens, pair_lut_ws, mid_o, B, Hq, Hk, D,
-                 block_size, max_blocks_per_seq, cache_block_stride, num_kv_splits, layout,
-                 attn_scale, sinks};
-    a.query_dtype = query_dtype;
-    const int waves = check_stage1(a) == TQ4_OK ? decode_waves(a) : 0;
-    if (waves > 0) {
-        if (!out || !lse || !query || !rot_t)
-            return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
-        if (out_dtype != TQ4_F32 && out_dtype != TQ4_BF16 && out_dtype != TQ4_F16)
-            return fail(TQ4_E_INVALID, "tq4_full_decode: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
-        a.out = out;
-        a.out_dtype = out_dtype;
-        a.lse = lse;
-        if (waves == 1 && rot_applies(a) && aligned(query, 16)) {
-            // one launch: the workgroup of each sequence rotates its query into LDS (the
-            // workspaces q_rot_ws and pair_lut_ws are not written)
-            a.query = query;
-            a.rot_t = rot_t;
-            a.lut = centroids;
-            return run_stage1(a, TQ4_KERNEL_XDL, st);
-        }
-        const int rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
-        return rc ? rc : run_parts(a, waves, st);
-    }
-    // one launch rotates the query and writes the pair LUT
-    int rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, centroids, pair_lut_ws, st);
-    if (rc)
-        return rc;
-    rc = run_stage1(a, TQ4_KERNEL_AUTO, st);
-    if (rc)
-        return rc;
-    return tq4_stage2(mid_o, seq_lens, out, out_dtype, lse, B, Hq, D, a.S, stream);
+    return full_decode(query, query_dtype, rot_t, centroids, kv_cache, block_table, seq_lens, q_rot_ws, pair_lut_ws,
+                       mid_o, true, out, out_dtype, lse, B, Hq, Hk, D, block_size, max_blocks_per_seq,
+                       cache_block_stride, num_kv_splits, layout, attn_scale, sinks,
+                       reinterpret_cast<hipStream_t>(stream));
 }
 
 int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_t, const float *centroids,
@@ -671,10 +780,6 @@ int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_
                                        "(8/4, 3/4, 3/3)", key_bits, value_bits);
     if (!query || !out || !lse || (!fp8 && (!rot_t || !centroids)))
         return fail(TQ4_E_INVALID, "tq4_full_decode_preset: null pointer argument");
-    if (query_dtype != TQ4_F32 && query_dtype != TQ4_BF16 && query_dtype != TQ4_F16)
-        return fail(TQ4_E_INVALID, "tq4_full_decode_preset: query_dtype must be 0, 1 or 2");
-    if (out_dtype != TQ4_F32 && out_dtype != TQ4_BF16 && out_dtype != TQ4_F16)
-        return fail(TQ4_E_INVALID, "tq4_full_decode_preset: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     Stage1Args a{fp8 ? static_cast<const float *>(query) : q_rot_ws, kv_cache, block_table, seq_lens, centroids,
                  mid_o, B, Hq, Hk, D, block_size, max_blocks_per_seq, cache_block_stride, num_kv_splits, layout,
@@ -682,23 +787,19 @@ int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_
     a.key_fp8 = fp8;
     a.key_bits = fp8 ? 0 : key_bits;
     a.value_bits = value_bits;
-    a.query_dtype = query_dtype;
-    int rc = check_stage1(a);
+    int rc = check_step("tq4_full_decode_preset", query, query_dtype, out_dtype);
+    if (rc == TQ4_OK)
+        rc = check_stage1(a);
     if (rc)
         return rc;
-    const int waves = decode_waves(a);
-    if (fp8 && waves == 0 && query_dtype != TQ4_F32)
+    if (mfma_applies(a))
+        return run_step(a, StepIo{query, query_dtype, rot_t, q_rot_ws, centroids, out, out_dtype, lse}, true, st);
+    if (fp8 && query_dtype != TQ4_F32)
         return fail(TQ4_E_UNSUPPORTED, "tq4_full_decode_preset: FP8 keys on the VALU kernel take an fp32 query");
     if (!fp8) {
         rc = rotate_query(query, query_dtype, rot_t, q_rot_ws, B * Hq, D, nullptr, nullptr, st);
         if (rc)
             return rc;
-    }
-    if (waves > 0) {
-        a.out = out;
-        a.out_dtype = out_dtype;
-        a.lse = lse;
-        return run_parts(a, waves, st);
     }
     rc = run_stage1(a, TQ4_KERNEL_AUTO, st);
     if (rc)
@@ -721,8 +822,8 @@ int tq4_full_decode_noalloc(const void *query, int query_dtype, const float *rot
     int rc = scratch_address(&base);
     if (rc)
         return rc;
-    // scratch layout: pair LUT | q_rot [B, Hq, D] | mid_o [B, Hq, S, D + 1] (only when Stage1
-    // runs more than one split per sequence), each 256-byte aligned
+    // scratch layout: pair LUT | q_rot [B, Hq, D] | mid_o [B, Hq, S, D + 1] (only where it is
+    // used), each 256-byte aligned
     unsigned char *bytes = static_cast<unsigned char *>(base);
     const size_t lut_bytes = round_up(256 * 2 * sizeof(float), kScratchAlign);
     const size_t q_bytes = round_up((size_t)B * Hq * D * sizeof(float), kScratchAlign);
@@ -734,17 +835,26 @@ int tq4_full_decode_noalloc(const void *query, int query_dtype, const float *rot
     rc = check_stage1(a);  // invalid arguments report their own error, not a workspace size
     if (rc)
         return rc;
-    const bool one_wave = decode_waves(a) == 1;  // the step then writes no part rows
-    const size_t mid_bytes = one_wave ? 0 : (size_t)B * Hq * num_kv_splits * (D + 1) * sizeof(float);
+    // batches whose (sequence, head part) pairs have fewer than two waves each are taken
+    // whatever the rows need: where they do not fit, a workgroup takes a whole sequence
+    const int64_t pairs = (int64_t)Hk * xdl_parts(a) * B, held = step_waves_held();
+    const bool one_wave =
+        mfma_applies(a) && (num_kv_splits == 1 || (pairs + held - 1) / held * held < 2 * pairs);
+    const size_t row_bytes = (size_t)B * Hq * num_kv_splits * (D + 1) * sizeof(float);
+    const bool have_parts = lut_bytes + q_bytes + row_bytes <= kScratchBytes;
+    const size_t mid_bytes = one_wave && !have_parts ? 0 : row_bytes;
     const size_t need = lut_bytes + q_bytes + mid_bytes;
     if (need > kScratchBytes)
         return fail(TQ4_E_INVALID,
                     "tq4_full_decode_noalloc: B=%d Hq=%d S=%d needs %zu bytes of workspace (q_rot %zu, "
                     "mid_o %zu), the library's scratch holds %zu",
                     B, Hq, num_kv_splits, need, q_bytes, mid_bytes, kScratchBytes);
-    return tq4_full_decode(query, query_dtype, rot_t, centroids, kv_cache, block_table, seq_lens, q_rot, lut,
-                           mid_o, out, out_dtype, lse, B, Hq, Hk, D, block_size, max_blocks_per_seq,
-                           cache_block_stride, num_kv_splits, layout, attn_scale, sinks, stream);
+    if (!centroids)
+        return fail(TQ4_E_INVALID, "tq4_full_decode: null pointer argument");
+    return full_decode(query, query_dtype, rot_t, centroids, kv_cache, block_table, seq_lens, q_rot, lut, mid_o,
+                       have_parts, out, out_dtype, lse, B, Hq, Hk, D, block_size, max_blocks_per_seq,
+                       cache_block_stride, num_kv_splits, layout, attn_scale, sinks,
+                       reinterpret_cast<hipStream_t>(stream));
 }
 
 int tq4_store(const void *key, const void *value, int dtype, const int32_t *slot_mapping,
