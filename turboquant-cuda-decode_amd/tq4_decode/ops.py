@@ -32,6 +32,10 @@ from .layout import AOS, AOS_HEAD_MAJOR, LAYOUTS, SOA, slot_bytes, slot_bytes_fp
 KERNELS = {"auto": 0, "simple": 1, "xdl": 3}
 DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 HEAD_DIM = 128
+_KEY_SHAPE = f"key must be [N, Hk, {HEAD_DIM}]"
+_QUERY_SHAPE = f"query must be [B, Hq, {HEAD_DIM}]"
+_HEAD_DIM = f"requires D={HEAD_DIM}"
+_ROTATION_SHAPE = f"rotation must be [{HEAD_DIM}, {HEAD_DIM}]"
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -39,19 +43,38 @@ def _require(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
+# The checks below run on every call, at about the cost of a launch: they format their messages
+# only when they fail, and ask for the raw stream handle instead of a Stream object (a decode
+# step of one short sequence: 21.8 us with eager messages and views made anew, 12.7 so).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _check_tensor(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
+    if t.is_cuda and t.dtype is dtype and t.is_contiguous():
+        return
     _require(t.is_cuda, f"{name} must be CUDA")
     _require(t.dtype == dtype, f"{name} must be {str(dtype).replace('torch.', '')}")
     _require(t.is_contiguous(), f"{name} must be contiguous")
 
 
+def _same_device(first: torch.Tensor, *others: torch.Tensor) -> bool:
+    dev = first.device
+    for t in others:
+        if t.device != dev:
+            return False
+    return True
+
+
 def _layout_id(layout) -> int:
     if isinstance(layout, str):
-        _require(layout in LAYOUTS, f"layout must be one of {sorted(LAYOUTS)}")
+        if layout not in LAYOUTS:
+            raise RuntimeError(f"layout must be one of {sorted(LAYOUTS)}")
         return LAYOUTS[layout]
     _require(layout in (SOA, AOS), "layout must be 0 (SoA) or 1 (AoS)")
     return int(layout)
@@ -77,15 +100,13 @@ def _cache_geometry(kv_cache: torch.Tensor, slot_want: int, layout, preset: str 
 def block_geometry(shape, strides, slot_want: int, layout, preset: str = ""):
     """The stride rules of ``_cache_geometry`` for a 4-D uint8 ``shape`` / ``strides``."""
     nb, bs, hk, slot = shape
-    _require(slot == slot_want, f"requires slot_size={slot_want}{preset}")
+    if slot != slot_want:
+        raise RuntimeError(f"requires slot_size={slot_want}{preset}")
     s0, s1, s2, s3 = strides
-
-    def same(size, got, want):  # a dimension of size 1 has no meaningful stride
-        return size == 1 or got == want
-
-    _require(same(slot, s3, 1), "kv_cache: the slot bytes must be contiguous (stride(3) == 1)")
-    position_major = same(bs, s1, hk * slot) and same(hk, s2, slot)
-    head_major = same(bs, s1, slot) and same(hk, s2, bs * slot)
+    # (a dimension of size 1 has no meaningful stride)
+    _require(s3 == 1 or slot == 1, "kv_cache: the slot bytes must be contiguous (stride(3) == 1)")
+    position_major = (s1 == hk * slot or bs == 1) and (s2 == slot or hk == 1)
+    head_major = (s1 == slot or bs == 1) and (s2 == bs * slot or hk == 1)
     _require(position_major or head_major,
              "kv_cache: each block must be a contiguous [block_size, Hk, slot] block or the "
              "transpose(1, 2) view of a contiguous [Hk, block_size, slot] block")
@@ -129,7 +150,7 @@ def stage1(q_rot, kv_cache, block_table, seq_lens, pair_lut, mid_o=None, *, num_
         _check_tensor(t, n, dt)
     _require(q_rot.dim() == 3, "q_rot must be [B, Hq, D]")
     B, Hq, D = q_rot.shape
-    _require(D == HEAD_DIM, f"requires D={HEAD_DIM}")
+    _require(D == HEAD_DIM, _HEAD_DIM)
     bs, Hk, stride, lid = _cache_geometry(kv_cache, slot_bytes(D), layout)
     _require(Hq % Hk == 0, "Hq must be a multiple of Hk")
     _require(block_table.dim() == 2 and block_table.size(0) == B, "block_table batch mismatch")
@@ -141,13 +162,13 @@ def stage1(q_rot, kv_cache, block_table, seq_lens, pair_lut, mid_o=None, *, num_
         mid_o = torch.empty(B, Hq, num_kv_splits, D + 1, dtype=torch.float32, device=q_rot.device)
     _check_tensor(mid_o, "mid_o", torch.float32)
     S = mid_o.size(2)
-    _require(mid_o.dim() == 4 and tuple(mid_o.shape) == (B, Hq, S, D + 1),
-             f"mid_o must be [B,{Hq},S,{D + 1}]")
+    if not (mid_o.dim() == 4 and tuple(mid_o.shape) == (B, Hq, S, D + 1)):
+        raise RuntimeError(f"mid_o must be [B,{Hq},S,{D + 1}]")
     _require(num_kv_splits is None or num_kv_splits == S, "mid_o split count mismatch")
-    devs = {t.device for t in (q_rot, kv_cache, block_table, seq_lens, pair_lut, mid_o)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    _require(_same_device(q_rot, kv_cache, block_table, seq_lens, pair_lut, mid_o), "all tensors must be on the same device")
     scale = 1.0 / math.sqrt(D) if attn_scale is None else float(attn_scale)
-    _require(kernel in KERNELS, f"kernel must be one of {sorted(KERNELS)}")
+    if kernel not in KERNELS:
+        raise RuntimeError(f"kernel must be one of {sorted(KERNELS)}")
     sinks_ptr = _check_sinks(sinks, Hq, q_rot.device)
     rc = _lib.load().tq4_stage1_ex(
         q_rot.data_ptr(), kv_cache.data_ptr(), block_table.data_ptr(), seq_lens.data_ptr(),
@@ -184,7 +205,7 @@ def rotate_query(query, rotation_t, q_rot=None):
     _require(query.is_cuda and query.is_contiguous() and query.dtype in DTYPES, "invalid query")
     _check_tensor(rotation_t, "rotation_t", torch.float32)
     _require(query.size(-1) == HEAD_DIM and tuple(rotation_t.shape) == (HEAD_DIM, HEAD_DIM),
-             f"requires D={HEAD_DIM}")
+             _HEAD_DIM)
     if q_rot is None:
         q_rot = torch.empty(query.shape, dtype=torch.float32, device=query.device)
     _check_tensor(q_rot, "q_rot", torch.float32)
@@ -208,12 +229,12 @@ def store(key, value, kv_cache, slot_mapping, rotation_t, midpoints, centroids=N
     _require(key.is_cuda and key.dtype in DTYPES and key.is_contiguous(), "invalid key")
     _require(value.dtype == key.dtype and value.is_contiguous() and value.shape == key.shape,
              "value must match key (shape, dtype, contiguous)")
-    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, f"key must be [N, Hk, {HEAD_DIM}]")
+    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, _KEY_SHAPE)
     _check_tensor(slot_mapping, "slot_mapping", torch.int32)
     _check_tensor(rotation_t, "rotation_t", torch.float32)
     _check_tensor(midpoints, "midpoints", torch.float32)
     _require(midpoints.numel() == 15, "4-bit keys need 15 midpoints")
-    _require(tuple(rotation_t.shape) == (HEAD_DIM, HEAD_DIM), f"rotation must be [{HEAD_DIM}, {HEAD_DIM}]")
+    _require(rotation_t.shape == (HEAD_DIM, HEAD_DIM), _ROTATION_SHAPE)
     if norm_correction:
         _require(centroids is not None, "norm_correction=True requires centroids")
     if centroids is not None:
@@ -223,8 +244,7 @@ def store(key, value, kv_cache, slot_mapping, rotation_t, midpoints, centroids=N
     bs, hk, stride, lid = _cache_geometry(kv_cache, slot_bytes(D), layout)
     _require(hk == Hk, "kv_cache must be [blocks, block_size, Hk, slot]")
     _require(slot_mapping.numel() == N, "slot_mapping must have one entry per token")
-    devs = {t.device for t in (key, value, kv_cache, slot_mapping, rotation_t, midpoints)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    _require(_same_device(key, value, kv_cache, slot_mapping, rotation_t, midpoints), "all tensors must be on the same device")
     rc = _lib.load().tq4_store(
         key.data_ptr(), value.data_ptr(), DTYPES[key.dtype], slot_mapping.data_ptr(),
         rotation_t.data_ptr(), midpoints.data_ptr(),
@@ -242,7 +262,7 @@ def stage1_fp8(query, kv_cache, block_table, seq_lens, mid_o=None, *, num_kv_spl
     for t, n, dt in ((query, "query", torch.float32), (block_table, "block_table", torch.int32),
                      (seq_lens, "seq_lens", torch.int32)):
         _check_tensor(t, n, dt)
-    _require(query.dim() == 3 and query.size(2) == HEAD_DIM, f"query must be [B, Hq, {HEAD_DIM}]")
+    _require(query.dim() == 3 and query.size(2) == HEAD_DIM, _QUERY_SHAPE)
     B, Hq, D = query.shape
     bs, Hk, stride, lid = _cache_geometry(kv_cache, slot_bytes_fp8(D), layout, " (FP8 keys)")
     _require(Hq % Hk == 0, "Hq must be a multiple of Hk")
@@ -254,9 +274,9 @@ def stage1_fp8(query, kv_cache, block_table, seq_lens, mid_o=None, *, num_kv_spl
         mid_o = torch.empty(B, Hq, num_kv_splits, D + 1, dtype=torch.float32, device=query.device)
     _check_tensor(mid_o, "mid_o", torch.float32)
     S = mid_o.size(2)
-    _require(tuple(mid_o.shape) == (B, Hq, S, D + 1), f"mid_o must be [B,{Hq},S,{D + 1}]")
-    devs = {t.device for t in (query, kv_cache, block_table, seq_lens, mid_o)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    if mid_o.shape != (B, Hq, S, D + 1):
+        raise RuntimeError(f"mid_o must be [B,{Hq},S,{D + 1}]")
+    _require(_same_device(query, kv_cache, block_table, seq_lens, mid_o), "all tensors must be on the same device")
     scale = 1.0 / math.sqrt(D) if attn_scale is None else float(attn_scale)
     _require(kernel in ("auto", "xdl", "simple"), "kernel must be auto, xdl or simple")
     rc = _lib.load().tq4_stage1_fp8_ex(
@@ -273,14 +293,13 @@ def store_fp8(key, value, kv_cache, slot_mapping, *, layout="soa"):
     _require(key.is_cuda and key.dtype in DTYPES and key.is_contiguous(), "invalid key")
     _require(value.dtype == key.dtype and value.is_contiguous() and value.shape == key.shape,
              "value must match key (shape, dtype, contiguous)")
-    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, f"key must be [N, Hk, {HEAD_DIM}]")
+    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, _KEY_SHAPE)
     _check_tensor(slot_mapping, "slot_mapping", torch.int32)
     N, Hk, D = key.shape
     bs, hk, stride, lid = _cache_geometry(kv_cache, slot_bytes_fp8(D), layout, " (FP8 keys)")
     _require(hk == Hk, "kv_cache must be [blocks, block_size, Hk, slot]")
     _require(slot_mapping.numel() == N, "slot_mapping must have one entry per token")
-    devs = {t.device for t in (key, value, kv_cache, slot_mapping)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    _require(_same_device(key, value, kv_cache, slot_mapping), "all tensors must be on the same device")
     rc = _lib.load().tq4_store_fp8(
         key.data_ptr(), value.data_ptr(), DTYPES[key.dtype], slot_mapping.data_ptr(),
         kv_cache.data_ptr(), N, Hk, D, bs, stride, lid, _stream(key.device))
@@ -299,13 +318,16 @@ def stage1_preset(q_rot, kv_cache, block_table, seq_lens, centroids, mid_o=None,
     centroids; returns ``mid_o [B, Hq, S, D+1]``.  ``kernel``: "auto" (3/4 and 3/3 on the
     16x16x32 MFMA kernel where it applies, 4/4 and other shapes on the VALU kernel), "xdl" or
     "simple"."""
-    _require((key_bits, value_bits) in PRESETS, f"key/value bits must be one of {PRESETS}")
+    if (key_bits, value_bits) not in PRESETS:
+        raise RuntimeError(f"key/value bits must be one of {PRESETS}")
     for t, n, dt in ((q_rot, "q_rot", torch.float32), (block_table, "block_table", torch.int32),
                      (seq_lens, "seq_lens", torch.int32), (centroids, "centroids", torch.float32)):
         _check_tensor(t, n, dt)
-    _require(q_rot.dim() == 3 and q_rot.size(2) == HEAD_DIM, f"q_rot must be [B, Hq, {HEAD_DIM}]")
+    if not (q_rot.dim() == 3 and q_rot.size(2) == HEAD_DIM):
+        raise RuntimeError(f"q_rot must be [B, Hq, {HEAD_DIM}]")
     B, Hq, D = q_rot.shape
-    _require(centroids.numel() == 1 << key_bits, f"{key_bits}-bit keys need {1 << key_bits} centroids")
+    if centroids.numel() != 1 << key_bits:
+        raise RuntimeError(f"{key_bits}-bit keys need {1 << key_bits} centroids")
     bs, Hk, stride, lid = _cache_geometry(kv_cache, slot_bytes_preset(D, key_bits, value_bits), layout)
     _require(Hq % Hk == 0, "Hq must be a multiple of Hk")
     _require(block_table.dim() == 2 and block_table.size(0) == B, "block_table batch mismatch")
@@ -316,9 +338,9 @@ def stage1_preset(q_rot, kv_cache, block_table, seq_lens, centroids, mid_o=None,
         mid_o = torch.empty(B, Hq, num_kv_splits, D + 1, dtype=torch.float32, device=q_rot.device)
     _check_tensor(mid_o, "mid_o", torch.float32)
     S = mid_o.size(2)
-    _require(tuple(mid_o.shape) == (B, Hq, S, D + 1), f"mid_o must be [B,{Hq},S,{D + 1}]")
-    devs = {t.device for t in (q_rot, kv_cache, block_table, seq_lens, centroids, mid_o)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    if mid_o.shape != (B, Hq, S, D + 1):
+        raise RuntimeError(f"mid_o must be [B,{Hq},S,{D + 1}]")
+    _require(_same_device(q_rot, kv_cache, block_table, seq_lens, centroids, mid_o), "all tensors must be on the same device")
     scale = 1.0 / math.sqrt(D) if attn_scale is None else float(attn_scale)
     _require(kernel in ("auto", "xdl", "simple"), "kernel must be auto, xdl or simple")
     rc = _lib.load().tq4_stage1_preset_ex(
@@ -334,28 +356,30 @@ def store_preset(key, value, kv_cache, slot_mapping, rotation_t, midpoints, cent
                  key_bits, value_bits, layout="soa", norm_correction=True):
     """Writer of the bit-width presets: K index = number of the ``2^key_bits - 1``
     ``midpoints`` <= y, V codes at ``value_bits``; otherwise as ``store``."""
-    _require((key_bits, value_bits) in PRESETS, f"key/value bits must be one of {PRESETS}")
+    if (key_bits, value_bits) not in PRESETS:
+        raise RuntimeError(f"key/value bits must be one of {PRESETS}")
     _require(key.is_cuda and key.dtype in DTYPES and key.is_contiguous(), "invalid key")
     _require(value.dtype == key.dtype and value.is_contiguous() and value.shape == key.shape,
              "value must match key (shape, dtype, contiguous)")
-    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, f"key must be [N, Hk, {HEAD_DIM}]")
+    _require(key.dim() == 3 and key.size(2) == HEAD_DIM, _KEY_SHAPE)
     _check_tensor(slot_mapping, "slot_mapping", torch.int32)
     _check_tensor(rotation_t, "rotation_t", torch.float32)
     _check_tensor(midpoints, "midpoints", torch.float32)
     n_mid = (1 << key_bits) - 1
-    _require(midpoints.numel() == n_mid, f"{key_bits}-bit keys need {n_mid} midpoints")
-    _require(tuple(rotation_t.shape) == (HEAD_DIM, HEAD_DIM), f"rotation must be [{HEAD_DIM}, {HEAD_DIM}]")
+    if midpoints.numel() != n_mid:
+        raise RuntimeError(f"{key_bits}-bit keys need {n_mid} midpoints")
+    _require(rotation_t.shape == (HEAD_DIM, HEAD_DIM), _ROTATION_SHAPE)
     if norm_correction:
         _require(centroids is not None, "norm_correction=True requires centroids")
     if centroids is not None:
         _check_tensor(centroids, "centroids", torch.float32)
-        _require(centroids.numel() == n_mid + 1, f"{key_bits}-bit keys need {n_mid + 1} centroids")
+        if centroids.numel() != n_mid + 1:
+            raise RuntimeError(f"{key_bits}-bit keys need {n_mid + 1} centroids")
     N, Hk, D = key.shape
     bs, hk, stride, lid = _cache_geometry(kv_cache, slot_bytes_preset(D, key_bits, value_bits), layout)
     _require(hk == Hk, "kv_cache must be [blocks, block_size, Hk, slot]")
     _require(slot_mapping.numel() == N, "slot_mapping must have one entry per token")
-    devs = {t.device for t in (key, value, kv_cache, slot_mapping, rotation_t, midpoints)}
-    _require(len(devs) == 1, "all tensors must be on the same device")
+    _require(_same_device(key, value, kv_cache, slot_mapping, rotation_t, midpoints), "all tensors must be on the same device")
     rc = _lib.load().tq4_store_preset(
         key.data_ptr(), value.data_ptr(), DTYPES[key.dtype], slot_mapping.data_ptr(),
         rotation_t.data_ptr(), midpoints.data_ptr(),
@@ -391,7 +415,7 @@ def full_decode(query, rotation_t, kv_cache, block_table, seq_lens, centroids, n
         _check_tensor(t, n, dt)
     _require(query.dim() == 3, "query must be [B, Hq, D]")
     B, Hq, D = query.shape
-    _require(D == HEAD_DIM, f"requires D={HEAD_DIM}")
+    _require(D == HEAD_DIM, _HEAD_DIM)
     bs, Hk, stride, lid = _cache_geometry(kv_cache, slot_bytes(D), layout)
     out_dtype = query.dtype if out_dtype is None else out_dtype
     ws = workspace or DecodeWorkspace(B, Hq, num_kv_splits, query.device, out_dtype)
@@ -425,10 +449,11 @@ def _full_decode_preset(query, rotation_t, kv_cache, block_table, seq_lens, cent
     tensors = [query, kv_cache, block_table, seq_lens, ws.mid_o, ws.out, ws.lse]
     if not fp8:
         _check_tensor(rotation_t, "rotation_t", torch.float32)
-        _require(tuple(rotation_t.shape) == (D, D), f"requires D={HEAD_DIM}")
-        _require(centroids.numel() == 1 << key_bits, f"{key_bits}-bit keys need {1 << key_bits} centroids")
+        _require(tuple(rotation_t.shape) == (D, D), _HEAD_DIM)
+        if centroids.numel() != 1 << key_bits:
+            raise RuntimeError(f"{key_bits}-bit keys need {1 << key_bits} centroids")
         tensors += [rotation_t, centroids]
-    _require(len({t.device for t in tensors}) == 1, "all tensors must be on the same device")
+    _require(_same_device(*tensors), "all tensors must be on the same device")
     mfma = bs >= 16 and bs & (bs - 1) == 0 and stride % 16 == 0
     if fp8 and not (mfma and query.data_ptr() % 16 == 0):
         # the VALU kernel takes fp32 rows, and both take them aligned
@@ -448,6 +473,8 @@ def _buffer_view(buf, shape, dtype):
     """``buf`` cut to ``shape`` (leading sub-block) when it fits and stays contiguous."""
     if buf is None or buf.dtype != dtype or buf.dim() != len(shape):
         return None
+    if buf.shape == shape:  # the whole buffer, as a later call of the same shape finds it
+        return buf if buf.is_contiguous() else None
     if any(have < want for have, want in zip(buf.shape, shape)):
         return None
     view = buf[tuple(slice(0, n) for n in shape)]
@@ -506,19 +533,21 @@ def turboquant_decode_attention(query, kv_cache, block_table, seq_lens, Pi, cent
     ``turboquant_3bit_nc``, all on the 16x16x32 MFMA Stage1 where it applies (power-of-two
     blocks of 16 tokens or more), else the VALU kernel; 4-bit AoS without norm correction raises ``NotImplementedError``.
     """
-    _require(query.dim() == 3 and query.size(2) == HEAD_DIM, f"query must be [B, Hq, {HEAD_DIM}]")
+    _require(query.dim() == 3 and query.size(2) == HEAD_DIM, _QUERY_SHAPE)
     S = int(max_num_kv_splits)
     ws = _decode_buffers(query, S, buf_holder, mid_o_buf, output_buf, lse_buf)
     if key_fp8:
         _require(value_quant_bits == 4, "FP8 keys are built with 4-bit values")
-        _require(key_packed_size == HEAD_DIM, f"key_packed_size must be {HEAD_DIM} for FP8 keys")
+        if key_packed_size != HEAD_DIM:
+            raise RuntimeError(f"key_packed_size must be {HEAD_DIM} for FP8 keys")
         # the unrotated query (reference/soa_decode_v1.py:528-534)
         return _full_decode_preset(query.contiguous(), None, kv_cache, block_table, seq_lens, None, ws, key_bits=8,
                                    value_bits=4, layout=layout, attn_scale=scale, sinks=sinks)
-    _require((mse_bits, value_quant_bits) in PRESETS,
-             f"MSE key / value bits must be one of {PRESETS}")
+    if (mse_bits, value_quant_bits) not in PRESETS:
+        raise RuntimeError(f"MSE key / value bits must be one of {PRESETS}")
     want = HEAD_DIM * mse_bits // 8 + 2
-    _require(key_packed_size == want, f"key_packed_size must be {want}")
+    if key_packed_size != want:
+        raise RuntimeError(f"key_packed_size must be {want}")
     if layout == "aos" and not norm_correction:
         raise NotImplementedError("AoS decode is built with the norm correction (the _nc presets)")
     if PiT is None:
@@ -578,10 +607,11 @@ def triton_turboquant_store(key, value, kv_cache, slot_mapping, PiT, midpoints, 
 
 def _store_mse(key, value, kv_cache, slot_mapping, PiT, midpoints, mse_bits, key_packed_size,
                value_quant_bits, centroids, norm_correction, layout):
-    _require((mse_bits, value_quant_bits) in PRESETS,
-             f"MSE key / value bits must be one of {PRESETS}")
+    if (mse_bits, value_quant_bits) not in PRESETS:
+        raise RuntimeError(f"MSE key / value bits must be one of {PRESETS}")
     want = HEAD_DIM * mse_bits // 8 + 2
-    _require(key_packed_size == want, f"key_packed_size must be {want}")
+    if key_packed_size != want:
+        raise RuntimeError(f"key_packed_size must be {want}")
     if mse_bits == 4 and value_quant_bits == 4:
         store(key, value, kv_cache, slot_mapping, PiT, midpoints, centroids, layout=layout,
               norm_correction=norm_correction)
