@@ -35,13 +35,14 @@
 // Bucketize: the workgroup builds a cell table over the midpoints' span (kCells cells of
 // width w, about two spare cells each side, centred on y0 + kw with y0 = K w for an integer
 // K).  Cell k's window is [y0 + (k - 1/2)w - w/64, y0 + (k + 1/2)w + w/64]; its entry holds
-// the one midpoint inside the window (NaN if none), the number of midpoints below the
-// window, and c^2 at those two indices.  The cell of y is round(y / w - K), read straight
+// the one midpoint inside the window (NaN if none) and the number of midpoints below the
+// window.  The cell of y is round(y / w - K), read straight
 // from the bits of fma(y, 1/w, 1.5 * 2^23 - K) (the bias leaves the rounded integer in the
 // low mantissa bits) after a clamp to the table; a y whose computed cell is k lies inside
 // window k (the computed coordinate is off by < 1e-3 cells for |y| <= 1; beyond the span the
 // edge cells hold for every y), so count(midpoints <= y) = base + (y >= mid): one LDS read
-// and one compare per element instead of 15.  When some window holds two midpoints (a
+// and one compare per element instead of 15.  The entries are 8 bytes; c^2 of the index found
+// comes from a 16-entry table (no bank conflicts), in element order as before.  When some window holds two midpoints (a
 // codebook with a gap under ~w) the kernel counts all 15 instead.
 //
 // V codes: (v - min) * (1 / scale) is within 2^-18 of the fp32 quotient (v - min) / scale
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(kWave *W) __attribute__((amdgpu_waves_per_eu(W == k
     __shared__ __align__(16) _Float16 pt_lo[kHeadDim * kHeadDim];
     constexpr int kMids = (1 << KB) - 1;  // Lloyd-Max midpoints
     __shared__ float c2tab[16];
-    __shared__ __align__(16) float4 btab[kCells];
+    __shared__ __align__(16) float2 btab[kCells];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const int n = lane & 15, g = lane >> 4;
     const int tiles = (rows + kRows - 1) / kRows;
@@ -338,9 +339,8 @@ __global__ __launch_bounds__(kWave *W) __attribute__((amdgpu_waves_per_eu(W == k
             }
         }
         cell_ok = cell_ok && inside <= 1 && w > 0.f && w < __builtin_inff();
-        const int up = base < kMids ? base + 1 : kMids;
         // the midpoint is stored x 256, the scale of the rotation's results
-        btab[k] = float4{256.f * m_in, __builtin_bit_cast(float, base), c2_at(base), c2_at(up)};
+        btab[k] = float2{256.f * m_in, __builtin_bit_cast(float, base)};
     }
     const bool use_cells = __syncthreads_and(cell_ok) != 0;
     // biased cell coordinate y / w - K + 1.5 * 2^23 of y = acc / 256
@@ -368,15 +368,21 @@ __global__ __launch_bounds__(kWave *W) __attribute__((amdgpu_waves_per_eu(W == k
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                // v as one fp32 register value: otherwise the compiler may fold the product
-                // into one of the f16 casts (v_fma_mix, a single rounding) and not the other, and
-                // where the two roundings differ (the fp32 product on an f16 tie) hi + lo is off
-                // by an f16 ulp of x_hat * 16
-                float v = x[8 * kb + j] * rn;
-                asm("" : "+v"(v));
-                b_hi[kb][j] = (_Float16)v;
-                b_lo[kb][j] = (_Float16)(v - (float)b_hi[kb][j]);
+            for (int j = 0; j < 8; j += 2) {
+                float v0 = x[8 * kb + j] * rn, v1 = x[8 * kb + j + 1] * rn, l0, l1;
+                // The fp32 products stand in registers before the split (folded into one of the f16
+                // casts and not the other, hi + lo would be off by an f16 ulp on the products that are
+                // f16 ties), and the split is a packed cast and two mixed-precision fmas, v - hi
+                // exactly: 64 VALU fewer per tile than casting each hi twice and subtracting.
+                uint32_t h;
+                asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(v0), "v"(v1));
+                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(h), "v"(v0));
+                asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(l1) : "v"(h), "v"(v1));
+                const auto hp = __builtin_bit_cast(_Float16 __attribute__((ext_vector_type(2))), h);
+                b_hi[kb][j] = hp[0];
+                b_hi[kb][j + 1] = hp[1];
+                b_lo[kb][j] = (_Float16)l0;
+                b_lo[kb][j + 1] = (_Float16)l1;
             }
         // column block cb: MFMA row r <-> dim 32(r/4) + 4cb + r%4 (lane (n, g) feeds row n).
         // The operand reads are the same for every tile; an opaque base keeps them in the loop
@@ -408,16 +414,19 @@ __global__ __launch_bounds__(kWave *W) __attribute__((amdgpu_waves_per_eu(W == k
         if (use_cells) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
+                int idx[8];
 #pragma unroll
                 for (int j = 8 * q; j < 8 * q + 8; ++j) {
                     const float a = acc[j / 4][j % 4];
                     const float t = fminf(fmaxf(fmaf(a, inv_w, c0), kBias), kBias + (float)(kCells - 1));
-                    const float4 e = btab[__builtin_bit_cast(int, t) - __builtin_bit_cast(int, kBias)];
-                    const bool ge = a >= e.x;
-                    put_code<KB>(kw, j, (uint32_t)(__builtin_bit_cast(int, e.y) + (ge ? 1 : 0)));
-                    csq += ge ? e.w : e.z;
+                    const float2 e = btab[__builtin_bit_cast(int, t) - __builtin_bit_cast(int, kBias)];
+                    idx[j % 8] = __builtin_bit_cast(int, e.y) + (a >= e.x ? 1 : 0);
+                    put_code<KB>(kw, j, (uint32_t)idx[j % 8]);
                 }
-                // at most 8 table reads in flight (32 VGPRs)
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    csq += c2tab[idx[j]];
+                // at most 8 table reads in flight
                 asm volatile("" ::: "memory");
             }
         } else {
