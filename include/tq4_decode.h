@@ -146,7 +146,8 @@ int tq4_full_decode_preset(const void *query, int query_dtype, const float *rot_
  * Stage1 rows live in a 40 MiB device array the library holds on every GPU it runs on (from
  * its load until the process ends), so the call allocates nothing -- no hipMalloc, no
  * allocator.  Shapes whose workspace exceeds the array (2 KiB LUT + B*Hq*D*4 bytes of
- * q_rot + B*Hq*S*(D+1)*4 bytes of rows, these only while B * (head parts) <= half the waves the device holds) are
+ * q_rot + B*Hq*S*(D+1)*4 bytes of rows, the rows only when the (sequence, head part) pairs
+ * have two waves or more each) are
  * rejected with TQ4_E_INVALID.  Calls that overlap on one GPU share the array and race:
  * serialize them (one stream, or events).  Otherwise as tq4_full_decode.
  * No counterpart in the reference: for callers that cannot allocate (code under graph

@@ -546,12 +546,11 @@ int launch_store(const void *key, const void *value, int dtype, const int32_t *s
     return launch_status(what);
 }
 
-// Workspace of tq4_full_decode_noalloc in device memory the library owns: the pair LUT,
-// the rotated queries and (unless one split per sequence applies) the Stage1 rows.  One
-// copy per GPU the library runs on, held from the code object's load until the process
-// ends; calls that overlap on one GPU share it and race.  Nothing in it has to start at
-// zero: the rotation launch writes the LUT and q_rot before Stage1 reads them, and Stage2
-// reads only the rows of non-empty splits, which Stage1 writes.
+// Workspace of tq4_full_decode_noalloc in device memory the library owns: the pair LUT, the
+// rotated queries and the part (or Stage1) rows.  One copy per GPU the library runs on, held
+// from the code object's load until the process ends; calls that overlap on one GPU share it
+// and race.  Nothing in it has to start at zero: a merge reads only what the step wrote (and
+// discards what it requested ahead of the part count).
 constexpr size_t kScratchBytes = size_t(40) << 20;
 constexpr size_t kScratchAlign = 256;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];

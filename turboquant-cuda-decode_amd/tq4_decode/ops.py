@@ -403,7 +403,7 @@ class DecodeWorkspace:
 
 def full_decode(query, rotation_t, kv_cache, block_table, seq_lens, centroids, num_kv_splits, *,
                 layout="soa", out_dtype=None, attn_scale=None, workspace=None, sinks=None):
-    """Rotation + pair LUT + Stage1 + Stage2 in four launches; returns ``(out, lse)``.
+    """Query rotation, attention over the 4-bit cache and the merge; returns ``(out, lse)``.
 
     ``out`` is in ``out_dtype`` (default: the query dtype, as ``reference/soa_decode_v1.py:643``).
     """
@@ -517,8 +517,8 @@ def turboquant_decode_attention(query, kv_cache, block_table, seq_lens, Pi, cent
                                 lse_buf=None, buf_holder=None, max_num_kv_splits=32, sinks=None, *,
                                 layout="soa"):
     """The decode entry of the vLLM backend (``reference/soa_decode_v1.py:485-643``; AoS
-    ``reference/aos_decode.py:486-626``): ``q_rot = query @ PiT``, pair LUT, Stage1 over
-    ``max_num_kv_splits`` splits, Stage2; returns ``[B, Hq, D]`` in the query dtype.
+    ``reference/aos_decode.py:486-626``): ``q_rot = query @ PiT``, attention in at most
+    ``max_num_kv_splits`` parts per sequence, their merge; returns ``[B, Hq, D]`` in the query dtype.
 
     ``kv_cache`` is the contiguous ``[blocks, block_size, Hk, slot]`` cache or the backend's
     ``transpose(1, 2)`` view of its ``[blocks, Hk, block_size, slot]`` cache.  Caller buffers
