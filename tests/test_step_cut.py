@@ -20,7 +20,7 @@ def _const(text, name):
 
 
 SEGMENT, MIN_WAVE, WAVES = (_const(STEP, n) for n in ("kSegmentTiles", "kMinWaveTiles", "kStepWaves"))
-SHORT, MOST_PARTS = _const(HOST, "kShortTiles"), _const(HOST, "kMostParts")
+SHORT, MERGE, MOST_PARTS = (_const(HOST, n) for n in ("kShortTiles", "kMergeTiles", "kMostParts"))
 HELD = 256 * WAVES
 
 
@@ -37,7 +37,8 @@ def plan(batch, nvh, tiles, splits, most_vw, have_parts=True):
     if not full:
         while sw < WAVES and 2 * sw <= HELD // pairs:
             sw *= 2
-    if full or not have_parts or splits == 1 or up(tiles, sw) <= SHORT:
+    in_parts = max(MIN_WAVE, up(pairs * tiles, HELD))
+    if full or not have_parts or splits == 1 or up(tiles, sw) <= min(SHORT, in_parts + MERGE):
         return dict(vw=min(vw, WAVES // sw), sw=sw, nx=batch, per_seq=1, whole=True)
     sw = 1
     while sw < WAVES and HELD > pairs * sw * min(MOST_PARTS, splits - 1):

@@ -387,14 +387,20 @@ StepPlan step_plan(const Stage1Args &a, bool have_parts) {
     while (vw < most_vw && nvh % (2 * vw) == 0)
         vw *= 2;
     // whole: one wave per pair fills at least 9/10 of every round, so cutting further would only
-    // add the merge launch; or sequences so short that the waves a pair can have leave each at
-    // most kShortTiles tiles, where the merge costs more than an even cut of ragged lengths gives
-    constexpr int kShortTiles = 8;
+    // add the merge launch; or sequences so short that a wave has at most kShortTiles tiles, and at
+    // most kMergeTiles (about what the merge launch takes) more than it would have in parts.  Beyond
+    // kShortTiles ragged lengths lose more than the merge.  Whole / parts: 64 x 700 tokens 18.3 /
+    // 21.9 us (70 to 700: 18.0 / 21.9), 100 of 30 to 300 18.1 / 23.1 (11 and 10 tiles in either form);
+    // 1 x 1500 17.6 / 15.9 (12 against 4 tiles), 16 x 2000 20.6 / 18.7 (16 against 8).
+    constexpr int kShortTiles = 12;
+    constexpr int kMergeTiles = 5;
     const int64_t rounds = (pairs + held - 1) / held;
     const bool full = 10 * pairs >= 9 * rounds * held;
     int sw = full ? 1 : floor_pow2(held / pairs, tq4::xdl::kStepWaves);
-    if (full || !have_parts || (tiles + sw - 1) / sw <= kShortTiles)
-        return StepPlan{std::min(vw, tq4::xdl::kStepWaves / sw), sw, a.B, 1, true};
+    const int64_t wave_tiles = (tiles + sw - 1) / sw;
+    const int64_t parts_tiles = std::max<int64_t>(tq4::xdl::kMinWaveTiles, (pairs * tiles + held - 1) / held);
+    if (full || !have_parts || wave_tiles <= std::min<int64_t>(kShortTiles, parts_tiles + kMergeTiles))
+    return StepPlan{std::min(vw, tq4::xdl::kStepWaves / sw), sw, a.B, 1, true};
     // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
     // merge (and no more than there are rows); more waves than that cut ragged batches coarser
     // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
