@@ -9,7 +9,7 @@
 // sequences form one list, and workgroup x of the nx along the list takes an equal stretch of
 // it, across sequence ends if need be (a segment per sequence), so ragged batches and batch
 // sizes that do not divide the device keep every CU busy to the end.  The cut is worked out
-// here from seq_lens; the grid depends on shapes alone (step_plan in tq4_decode.hip).
+// in the kernel from seq_lens (step_cut.h); the grid depends on shapes alone (step_plan.h).
 //
 // Against num_splits rows of 129 floats per head this drops the mid_o traffic of all but one
 // row per workgroup, the split ends inside the stream, and for lengths that are not a multiple
@@ -25,27 +25,19 @@
 // launch starts, with every CU asking at once.
 #pragma once
 #include "stage1_xdl.h"
+#include "step_cut.h"
 
 namespace tq4 {
 namespace xdl {
 
-constexpr int kStepWaves = 8;              // waves per workgroup at most: two per SIMD of one CU
 constexpr int kQRowFloats = kHeadDim + 4;  // LDS row of a rotated query (rows 16 bytes apart in bank)
-// What a further segment costs a workgroup (block table, query, first loads), in tiles of its
-// stretch: a sequence counts this many tiles more than it has when the list is cut.  Measured,
-// 64 sequences of 512 to 8192 tokens, with 3 / 6 / 10 / 14 / 20: 79.7 / 78.1 / 76.3 / 75.3 / 77.3 us.
-constexpr int kSegmentTiles = 14;
-// Tiles whose block-table entries a wave keeps in LDS: a stream this long runs without a stop (a
-// stop, the block-table read and the refill of the ring, costs about 3 us).
-constexpr int kTableTiles = 512;
-constexpr int kMinWaveTiles = 4;  // a wave's stream is whole turns of the 4-slot ring anyway
 
-struct StepArgs {
+struct StepArgs : CutArgs {
     const void *query;         // ROT: the bf16 / fp16 query; else fp32 rows, already rotated (FP8 keys: q_dtype rows)
     const float *rot_t;        // [D, D] (ROT)
     const float *centroids;    // [16], 3-bit keys [8], FP8 keys null
     const uint8_t *cache;
-    const int32_t *block_table, *seq_lens;
+    const int32_t *block_table;
     const float *sinks;        // [Hq] or null
     float *parts;              // part rows (stage2.h); unused when whole
     void *out;
@@ -53,10 +45,9 @@ struct StepArgs {
     int64_t block_stride;
     float score_scale_log2;
     int q_dtype, out_dtype;
-    int batch, num_q_heads, num_kv_heads, block_size_log2, max_blocks, slot_pos, slot_head, num_splits;
+    int num_q_heads, num_kv_heads, block_size_log2, max_blocks, slot_pos, slot_head;
     int group, n_hp;           // q-heads per kv-head, head parts per kv-head
-    int vw, sw;                // head parts per workgroup and waves per head part (powers of two)
-    int per_seq;               // workgroups per sequence when all lengths are equal (0: fewer than one)
+    int vw;                    // head parts per workgroup (a power of two)
     int whole;                 // workgroup x holds sequence x and writes its output rows
 };
 
@@ -353,134 +344,6 @@ __device__ __forceinline__ void join_rows(const StepArgs &a, const RowSink &s, c
         if (lane == 0)
             sink_lse(a, s, h, mx + logf(wsum));
     }
-}
-
-// ---- The cut ------------------------------------------------------------------------------
-// Run i of n over `tiles` tiles: [first, first + count), the first tiles % n runs one longer.
-struct Run {
-    int first, count;
-};
-__device__ __forceinline__ Run run_of(int tiles, int n, int i) {
-    const int q = div_pos(tiles, n), r = tiles - q * n;
-    return Run{i * q + min(i, r), q + (i < r ? 1 : 0)};
-}
-
-// One workgroup's stretch of the list.  Sequences with tiles count tiles + kSegmentTiles; the
-// workgroup takes [x cell, (x + 1) cell) of that weight, and of sequence b, whose weight starts
-// at `start`, the tiles that fall in it after the first kSegmentTiles.
-struct Cut {
-    int b;           // current sequence (its batch index); >= batch: done
-    int len, tiles;
-    uint32_t start;  // weight of the sequences before b
-    uint32_t cell;   // weight per workgroup
-    Run run;         // the workgroup's tiles of sequence b
-    int p, n_parts;  // its part and the sequence's parts
-};
-__device__ __forceinline__ int tiles_of(int len) { return (max(len, 0) + 15) >> 4; }
-__device__ __forceinline__ uint32_t weight_of(int tiles) { return tiles > 0 ? (uint32_t)(tiles + kSegmentTiles) : 0u; }
-// Places the stretch in sequence c.b (c.len, c.start set).
-__device__ __forceinline__ void place(Cut &c, int x) {
-    c.tiles = tiles_of(c.len);
-    const int64_t first = (int64_t)c.start + kSegmentTiles, lo = (int64_t)x * c.cell - first;
-    const int t0 = (int)max(lo, (int64_t)0), t1 = (int)min(lo + (int64_t)c.cell, (int64_t)c.tiles);
-    c.run = Run{t0, max(t1 - t0, 0)};
-    if (c.run.count > 0) {
-        const int xf = (int)((uint32_t)first / c.cell), xl = (int)((uint32_t)(first + c.tiles - 1) / c.cell);
-        c.p = x - xf;
-        c.n_parts = xl - xf + 1;
-    }
-}
-// The next sequence in the stretch with tiles for this workgroup; false when there is none.
-__device__ __forceinline__ bool next_segment(Cut &c, const StepArgs &a, int x, bool inside) {
-    const uint64_t end = (uint64_t)(x + 1) * c.cell;
-    while (c.b < a.batch) {
-        if (inside) {  // leave sequence b
-            c.start += weight_of(tiles_of(c.len));
-            if (++c.b >= a.batch || c.start >= end)
-                return false;
-            c.len = a.seq_lens[c.b];
-        }
-        inside = true;
-        place(c, x);
-        if (c.run.count > 0)
-            return true;
-    }
-    return false;
-}
-// The first segment of workgroup x of nx.  `equal` (out): all lengths are the same and every
-// sequence takes the same number of workgroups, which then leave no segment cut.  len_lane:
-// seq_lens[lane], read by the caller.
-__device__ __forceinline__ bool first_segment(Cut &c, const StepArgs &a, int nx, int x, int lane, int len_lane,
-                                              bool &equal) {
-    const int32_t *sl = a.seq_lens;
-    const int len0 = __builtin_amdgcn_readfirstlane(len_lane);
-    uint32_t total = 0, most = 0, w0 = 0, s0 = 0;  // (w0, s0: the first 64 sequences' weights and their scan)
-    int l0 = 0;
-    bool same = true;
-    for (int c0 = 0; c0 < a.batch; c0 += kWave) {
-        const int len = c0 + lane >= a.batch ? 0 : c0 == 0 ? len_lane : sl[c0 + lane];
-        const int t = tiles_of(len);
-        const uint32_t w = weight_of(t), sc = wave_scan(w);
-        if (c0 == 0) {
-            l0 = len;
-            w0 = w;
-            s0 = sc;
-        }
-        total += (uint32_t)__builtin_amdgcn_readlane((int)sc, kWave - 1);
-        most = max(most, wave_max((uint32_t)t));
-        same = same && __ballot(c0 + lane < a.batch && len != len0) == 0;
-    }
-    if (most == 0)
-        return false;
-    const int least = kMinWaveTiles * a.sw;  // tiles below which a workgroup's waves run dry
-    uint32_t cell = max((uint32_t)div_pos((int)(total + nx - 1), nx), (uint32_t)least);
-    // at most num_splits parts: a sequence of T tiles touches at most (T - 1) / cell + 2 cells
-    if ((uint64_t)cell * (uint32_t)(a.num_splits - 1) < most)
-        cell = max(cell, (most + (uint32_t)a.num_splits - 2) / (uint32_t)(a.num_splits - 1));
-    equal = false;
-    if (same && a.per_seq > 0) {
-        const int k = min(min(a.per_seq, a.num_splits), (int)div_pos((int)most + least - 1, least));
-        // (3-bit keys, 48 sequences of 256 tiles on 256 workgroups: 5 each, 52 tiles, take 53.9 us;
-        // stretches of 51 take 56.7)
-        if ((uint32_t)div_pos((int)most + k - 1, k) <= cell + cell / 16) {
-            equal = true;
-            c.b = div_pos(x, k);
-            if (c.b >= a.batch)
-                return false;
-            c.len = len0;
-            c.tiles = (int)most;
-            c.p = x - c.b * k;
-            c.n_parts = k;
-            c.run = run_of(c.tiles, k, c.p);
-            return true;
-        }
-    }
-    c.cell = cell;
-    const uint64_t lo64 = (uint64_t)x * cell;
-    if (lo64 >= total)
-        return false;
-    const uint32_t lo = (uint32_t)lo64;
-    uint32_t carry = 0;
-    for (int c0 = 0; c0 < a.batch; c0 += kWave) {
-        int len = l0;
-        uint32_t w = w0, sc = s0;
-        if (c0 > 0) {
-            len = c0 + lane < a.batch ? sl[c0 + lane] : 0;
-            w = weight_of(tiles_of(len));
-            sc = wave_scan(w);
-        }
-        const uint32_t before = carry + sc - w;
-        const uint64_t hit = __ballot(w > 0 && lo >= before && lo < before + w);
-        if (hit) {
-            const int l = __builtin_ctzll(hit);
-            c.b = c0 + l;
-            c.len = __builtin_amdgcn_readlane(len, l);
-            c.start = (uint32_t)__builtin_amdgcn_readlane((int)before, l);
-            return next_segment(c, a, x, false);
-        }
-        carry += (uint32_t)__builtin_amdgcn_readlane((int)sc, kWave - 1);
-    }
-    return false;
 }
 
 // The kernel.  ROT: it rotates the (bf16 / fp16) query itself.  KF8 / KB3 / V3: the presets, as

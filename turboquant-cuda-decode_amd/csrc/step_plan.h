@@ -1,0 +1,82 @@
+// The full decode step's launch: constants, and how its workgroups are chosen from the shapes
+// alone.  Host code without HIP, so that tests compile it too.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace tq4 {
+namespace xdl {
+
+constexpr int kStepWaves = 8;  // waves per workgroup at most: two per SIMD of one CU
+// What a further segment costs a workgroup (block table, query, first loads), in tiles of its
+// stretch: a sequence counts this many tiles more than it has when the list is cut.  Measured,
+// 64 sequences of 512 to 8192 tokens, with 3 / 6 / 10 / 14 / 20: 79.7 / 78.1 / 76.3 / 75.3 / 77.3 us.
+constexpr int kSegmentTiles = 14;
+// Tiles whose block-table entries a wave keeps in LDS: a stream this long runs without a stop (a
+// stop, the block-table read and the refill of the ring, costs about 3 us).
+constexpr int kTableTiles = 512;
+constexpr int kMinWaveTiles = 4;  // a wave's stream is whole turns of the 4-slot ring anyway
+
+// How a step is cut into workgroups, from the shapes alone.
+struct StepPlan {
+    int vw, sw;    // head parts per workgroup, waves per head part
+    int nx;        // workgroups along the list of sequences
+    int per_seq;   // of them per sequence when lengths are equal
+    bool whole;    // one workgroup per sequence, which writes the output rows itself
+};
+inline int floor_pow2(int64_t x, int most) {
+    int p = 1;
+    while (p < most && 2 * p <= x)
+        p *= 2;
+    return p;
+}
+
+// What the plan depends on.
+struct StepShape {
+    int held;         // waves the device holds at once
+    int nvh;          // head parts of a sequence
+    int batch, max_blocks, block_size, num_splits;
+    bool whole_lines; // a head's records are whole 128-byte lines (4-bit SoA)
+};
+inline StepPlan step_plan(const StepShape &s, bool have_parts) {
+    const int held = s.held, nvh = s.nvh;
+    const int64_t pairs = (int64_t)nvh * s.batch;  // (sequence, head part) pairs
+    const int64_t tiles = ((int64_t)s.max_blocks * s.block_size + 15) / 16;  // of the longest sequence the table can hold
+    // eight head parts per workgroup for 4-bit SoA records (whole 128-byte lines), four for the others,
+    // whose neighbouring heads share lines: B64 x 4096 with 32 / 8 heads takes 66.0 (8) / 67.2 us
+    // (4), AoS 88.8 / 80.4, 3-bit B48 58.8 / 57.5; with two 70.3 to 73.6, 86 to 88 and 66.7
+    const int most_vw = s.whole_lines ? kStepWaves : kStepWaves / 2;
+    int vw = 1;
+    while (vw < most_vw && nvh % (2 * vw) == 0)
+        vw *= 2;
+    // whole: one wave per pair fills at least 9/10 of every round, so cutting further would only
+    // add the merge launch; or sequences so short that a wave has at most kShortTiles tiles, and at
+    // most kMergeTiles (about what the merge launch takes) more than it would have in parts.  Beyond
+    // kShortTiles ragged lengths lose more than the merge.  Whole / parts: 64 x 700 tokens 18.3 /
+    // 21.9 us (70 to 700: 18.0 / 21.9), 100 of 30 to 300 18.1 / 23.1 (11 and 10 tiles in either form);
+    // 1 x 1500 17.6 / 15.9 (12 against 4 tiles), 16 x 2000 20.6 / 18.7 (16 against 8).
+    constexpr int kShortTiles = 12;
+    constexpr int kMergeTiles = 5;
+    const int64_t rounds = (pairs + held - 1) / held;
+    const bool full = 10 * pairs >= 9 * rounds * held;
+    int sw = full ? 1 : floor_pow2(held / pairs, kStepWaves);
+    const int64_t wave_tiles = (tiles + sw - 1) / sw;
+    const int64_t parts_tiles = std::max<int64_t>(kMinWaveTiles, (pairs * tiles + held - 1) / held);
+    if (full || !have_parts || wave_tiles <= std::min<int64_t>(kShortTiles, parts_tiles + kMergeTiles))
+        return StepPlan{std::min(vw, kStepWaves / sw), sw, s.batch, 1, true};
+    // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
+    // merge (and no more than there are rows); more waves than that cut ragged batches coarser
+    // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
+    // 8192: 78.1 with one, 82.8 with two, 84.4 with four)
+    constexpr int kMostParts = 16;
+    sw = 1;
+    while (sw < kStepWaves && held > pairs * sw * std::min(kMostParts, s.num_splits - 1))
+        sw *= 2;
+    vw = std::min(vw, kStepWaves / sw);
+    const int64_t useful = s.batch * ((tiles + kMinWaveTiles * sw - 1) / (kMinWaveTiles * sw));
+    const int nx = (int)std::max<int64_t>(1, std::min<int64_t>(held / (vw * sw) / (nvh / vw), useful));
+    return StepPlan{vw, sw, nx, nx / s.batch, false};
+}
+
+}  // namespace xdl
+}  // namespace tq4

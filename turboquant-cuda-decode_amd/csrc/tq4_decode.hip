@@ -362,57 +362,11 @@ int step_waves_held() {
     return h;
 }
 
-// How a step is cut into workgroups, from the shapes alone.
-struct StepPlan {
-    int vw, sw;    // head parts per workgroup, waves per head part
-    int nx;        // workgroups along the list of sequences
-    int per_seq;   // of them per sequence when lengths are equal
-    bool whole;    // one workgroup per sequence, which writes the output rows itself
-};
-int floor_pow2(int64_t x, int most) {
-    int p = 1;
-    while (p < most && 2 * p <= x)
-        p *= 2;
-    return p;
-}
+using tq4::xdl::StepPlan;
 StepPlan step_plan(const Stage1Args &a, bool have_parts) {
-    const int held = step_waves_held(), nvh = a.Hk * xdl_parts(a);
-    const int64_t pairs = (int64_t)nvh * a.B;  // (sequence, head part) pairs
-    const int64_t tiles = ((int64_t)a.max_blocks * a.bs + 15) / 16;  // of the longest sequence the table can hold
-    // eight head parts per workgroup for 4-bit SoA records (whole 128-byte lines), four for the others,
-    // whose neighbouring heads share lines: B64 x 4096 with 32 / 8 heads takes 66.0 (8) / 67.2 us
-    // (4), AoS 88.8 / 80.4, 3-bit B48 58.8 / 57.5; with two 70.3 to 73.6, 86 to 88 and 66.7
-    const int most_vw = a.kl == 0 && !a.key_fp8 && a.key_bits == 0 ? tq4::xdl::kStepWaves : tq4::xdl::kStepWaves / 2;
-    int vw = 1;
-    while (vw < most_vw && nvh % (2 * vw) == 0)
-        vw *= 2;
-    // whole: one wave per pair fills at least 9/10 of every round, so cutting further would only
-    // add the merge launch; or sequences so short that a wave has at most kShortTiles tiles, and at
-    // most kMergeTiles (about what the merge launch takes) more than it would have in parts.  Beyond
-    // kShortTiles ragged lengths lose more than the merge.  Whole / parts: 64 x 700 tokens 18.3 /
-    // 21.9 us (70 to 700: 18.0 / 21.9), 100 of 30 to 300 18.1 / 23.1 (11 and 10 tiles in either form);
-    // 1 x 1500 17.6 / 15.9 (12 against 4 tiles), 16 x 2000 20.6 / 18.7 (16 against 8).
-    constexpr int kShortTiles = 12;
-    constexpr int kMergeTiles = 5;
-    const int64_t rounds = (pairs + held - 1) / held;
-    const bool full = 10 * pairs >= 9 * rounds * held;
-    int sw = full ? 1 : floor_pow2(held / pairs, tq4::xdl::kStepWaves);
-    const int64_t wave_tiles = (tiles + sw - 1) / sw;
-    const int64_t parts_tiles = std::max<int64_t>(tq4::xdl::kMinWaveTiles, (pairs * tiles + held - 1) / held);
-    if (full || !have_parts || wave_tiles <= std::min<int64_t>(kShortTiles, parts_tiles + kMergeTiles))
-    return StepPlan{std::min(vw, tq4::xdl::kStepWaves / sw), sw, a.B, 1, true};
-    // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
-    // merge (and no more than there are rows); more waves than that cut ragged batches coarser
-    // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
-    // 8192: 78.1 with one, 82.8 with two, 84.4 with four)
-    constexpr int kMostParts = 16;
-    sw = 1;
-    while (sw < tq4::xdl::kStepWaves && held > pairs * sw * std::min(kMostParts, a.S - 1))
-        sw *= 2;
-    vw = std::min(vw, tq4::xdl::kStepWaves / sw);
-    const int64_t useful = a.B * ((tiles + tq4::xdl::kMinWaveTiles * sw - 1) / (tq4::xdl::kMinWaveTiles * sw));
-    const int nx = (int)std::max<int64_t>(1, std::min<int64_t>(held / (vw * sw) / (nvh / vw), useful));
-    return StepPlan{vw, sw, nx, nx / a.B, false};
+    const bool whole_lines = a.kl == 0 && !a.key_fp8 && a.key_bits == 0;
+    return tq4::xdl::step_plan(
+        {step_waves_held(), a.Hk * xdl_parts(a), a.B, a.max_blocks, a.bs, a.S, whole_lines}, have_parts);
 }
 
 template <int LAYOUT, int G, bool ROT, bool KF8 = false, bool KB3 = false, bool V3 = false>
