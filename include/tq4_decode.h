@@ -111,7 +111,8 @@ int tq4_build_pair_lut(const float *centroids, float *pair_lut, int n_centroids,
  * tq4_stage1_ex (may be NULL).  query must be 16-byte aligned.  q_rot_ws (B*Hq*D floats),
  * pair_lut_ws (512 floats) and mid_o (B*Hq*num_kv_splits*(D+1) floats) are workspaces, their
  * contents after the call unspecified.  Where the 16x16x32 kernel applies, one launch rotates
- * the query (TQ4_F32 queries: a launch before it, into q_rot_ws) and runs the attention: with
+ * the query (TQ4_F32 queries, and head counts that leave workgroups of one or two waves: a
+ * launch before it, into q_rot_ws) and runs the attention: with
  * one workgroup per sequence it writes out / lse itself, else it leaves at most num_kv_splits
  * rows per sequence and head in mid_o, in a layout of its own, for a merge launch.  Other
  * shapes: rotation and pair LUT, Stage1, Stage2.

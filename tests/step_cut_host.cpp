@@ -121,12 +121,12 @@ void one_lane(int lane) {
 
 extern "C" {
 
-// out: vw, sw, nx, per_seq, whole
+// out: vw, sw, nx, per_seq, whole, rotates
 void host_step_plan(int held, int nvh, int batch, int max_blocks, int block_size, int num_splits, int whole_lines,
                     int have_parts, int *out) {
     const auto p = tq4::xdl::step_plan(
         {held, nvh, batch, max_blocks, block_size, num_splits, whole_lines != 0}, have_parts != 0);
-    out[0] = p.vw, out[1] = p.sw, out[2] = p.nx, out[3] = p.per_seq, out[4] = p.whole;
+    out[0] = p.vw, out[1] = p.sw, out[2] = p.nx, out[3] = p.per_seq, out[4] = p.whole, out[5] = p.rotates;
 }
 
 // The segments of workgroup x0 of n along the list, five ints each (sequence, first tile, end tile,

@@ -59,3 +59,16 @@ def test_the_host_build_sees_more_than_64_sequences_and_long_lists():
     """The carry past the first 64 sequences, and weights beyond 2^24 tiles."""
     for lens in ([16 * (1 + i % 7) for i in range(200)], [2 ** 24 * 3] * 5 + [1] * 70, [0] * 64 + [5000] * 70):
         check_cut(lens, 32, host.plan(len(lens), 8, up(max(lens), 16), 32))
+
+
+@pytest.mark.parametrize("nvh", [1, 2, 3, 4, 5, 6, 8, 12, 16])
+def test_small_workgroups_do_not_rotate_the_query(nvh):
+    """One or two waves would stage the rotation matrix in eight or four rounds for every segment.  Four
+    waves and more keep the rotation, and so does the one workgroup of a whole sequence."""
+    for batch in (1, 2, 8, 16, 64, 128, 256, 400):
+        for blocks, splits in ((20, 32), (256, 32), (2048, 16), (256, 2), (256, 1)):
+            for lines in (True, False):
+                p = host.plan(batch, nvh, blocks, splits, whole_lines=lines)
+                assert p.rotates == (p.vw * p.sw >= 4 or (p.whole and p.vw == nvh))
+    p = host.plan(64, nvh, 500, 32)  # 64 sequences of up to 8000 tokens: one wave per head part (two for one part)
+    assert p.rotates == (nvh % 4 == 0)

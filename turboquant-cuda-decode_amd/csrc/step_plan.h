@@ -15,6 +15,7 @@ constexpr int kSegmentTiles = 14;
 // Tiles whose block-table entries a wave keeps in LDS: a stream this long runs without a stop (a
 // stop, the block-table read and the refill of the ring, costs about 3 us).
 constexpr int kTableTiles = 512;
+constexpr int kRotateWaves = 4;   // least waves of a workgroup that rotates (StepPlan::rotates)
 constexpr int kMinWaveTiles = 4;  // a wave's stream is whole turns of the 4-slot ring anyway
 
 // How a step is cut into workgroups, from the shapes alone.
@@ -23,6 +24,14 @@ struct StepPlan {
     int nx;        // workgroups along the list of sequences
     int per_seq;   // of them per sequence when lengths are equal
     bool whole;    // one workgroup per sequence, which writes the output rows itself
+    // Its workgroups rotate a 16-bit query themselves.  Every segment stages all 64 KB of rot_t, 16
+    // columns per wave at a time: with one or two waves that is eight or four rounds of load, barrier
+    // and arithmetic, and the launch that rotates all rows first is faster, unless one workgroup
+    // has a whole sequence's heads and so stages rot_t once for it.  In the kernel / by the launch:
+    // 8 heads on 1 kv-head, 64 sequences of 500 to 8000 tokens (two waves): 40.0 / 31.6 us; 5 kv-heads,
+    // 256 x 2000 (one wave): 125.8 / 109.8; 6 kv-heads, 64 of 500 to 8000 (two): 73.3 / 67.1; 4 kv-heads
+    // (four waves): 48.7 / 48.7; 8 kv-heads, 64 x 4096 (eight): 68.1 / 70.6, AoS (four): 82.8 / 83.5.
+    bool rotates;
 };
 inline int floor_pow2(int64_t x, int most) {
     int p = 1;
@@ -62,8 +71,10 @@ inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     int sw = full ? 1 : floor_pow2(held / pairs, kStepWaves);
     const int64_t wave_tiles = (tiles + sw - 1) / sw;
     const int64_t parts_tiles = std::max<int64_t>(kMinWaveTiles, (pairs * tiles + held - 1) / held);
-    if (full || !have_parts || wave_tiles <= std::min<int64_t>(kShortTiles, parts_tiles + kMergeTiles))
-        return StepPlan{std::min(vw, kStepWaves / sw), sw, s.batch, 1, true};
+    if (full || !have_parts || wave_tiles <= std::min<int64_t>(kShortTiles, parts_tiles + kMergeTiles)) {
+        vw = std::min(vw, kStepWaves / sw);
+        return StepPlan{vw, sw, s.batch, 1, true, vw * sw >= kRotateWaves || vw == nvh};
+    }
     // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
     // merge (and no more than there are rows); more waves than that cut ragged batches coarser
     // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
@@ -75,7 +86,7 @@ inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     vw = std::min(vw, kStepWaves / sw);
     const int64_t useful = s.batch * ((tiles + kMinWaveTiles * sw - 1) / (kMinWaveTiles * sw));
     const int nx = (int)std::max<int64_t>(1, std::min<int64_t>(held / (vw * sw) / (nvh / vw), useful));
-    return StepPlan{vw, sw, nx, nx / s.batch, false};
+    return StepPlan{vw, sw, nx, nx / s.batch, false, vw * sw >= kRotateWaves};
 }
 
 }  // namespace xdl

@@ -406,7 +406,7 @@ int run_step(const Stage1Args &a, const StepIo &io, bool have_parts, hipStream_t
     s.query = io.query;
     s.q_dtype = io.query_dtype;
     if (!a.key_fp8) {
-        if (io.query_dtype == TQ4_F32) {  // the in-kernel rotation takes 16-bit queries
+        if (io.query_dtype == TQ4_F32 || !plan.rotates) {  // the in-kernel rotation takes 16-bit queries
             const int rc = rotate_query(io.query, io.query_dtype, io.rot_t, io.q_rot_ws, a.B * a.Hq, a.D, nullptr,
                                         nullptr, st);
             if (rc)
