@@ -72,3 +72,28 @@ def test_small_workgroups_do_not_rotate_the_query(nvh):
                 assert p.rotates == (p.vw * p.sw >= 4 or (p.whole and p.vw == nvh))
     p = host.plan(64, nvh, 500, 32)  # 64 sequences of up to 8000 tokens: one wave per head part (two for one part)
     assert p.rotates == (nvh % 4 == 0)
+
+
+@pytest.mark.parametrize("batch,nvh,lo,hi,table,splits,most", [
+    (16, 1, 30, 500, 2048, 32, 1),    # short sequences under a backend's wide table: a workgroup each
+    (64, 8, 250, 4000, 250, 2, 1),    # two rows per sequence leave no room for stretches
+    (64, 8, 3900, 4096, 256, 32, 4),
+    (16, 8, 30, 500, 2048, 32, 8),
+])
+def test_sequences_have_workgroups_of_their_own(batch, nvh, lo, hi, table, splits, most):
+    """Where that is no slower no workgroup takes a second segment, and no sequence more than `most`."""
+    lens = [lo + (hi - lo) * i // (batch - 1) for i in range(batch)]
+    p = host.plan(batch, nvh, table, splits)
+    assert not p.whole
+    cut = [host.segments(lens, splits, p, x) for x in range(p.nx)]
+    assert max(len(c) for c in cut) == 1
+    assert max(s[4] for c in cut for s in c) == most
+    check_cut(lens, splits, p)
+
+
+@pytest.mark.parametrize("batch,lo,hi", [(64, 512, 8192), (140, 4000, 4000), (200, 100, 2000), (100, 200, 3000)])
+def test_uneven_batches_are_cut_into_stretches(batch, lo, hi):
+    lens = [lo + (hi - lo) * i // (batch - 1) for i in range(batch)]
+    p = host.plan(batch, 8, up(hi, 16), 32)
+    assert not p.whole
+    assert max(len(host.segments(lens, 32, p, x)) for x in range(p.nx)) > 1

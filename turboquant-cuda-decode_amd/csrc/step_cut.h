@@ -16,7 +16,7 @@ struct CutArgs {
     const int32_t *seq_lens;
     int batch, num_splits;
     int sw;       // waves per head part (a power of two)
-    int per_seq;  // workgroups per sequence when all lengths are equal (0: fewer than one)
+    int per_seq;  // workgroups there are per sequence (0: fewer than one)
 };
 
 // Run i of n over `tiles` tiles: [first, first + count), the first tiles % n runs one longer.
@@ -70,16 +70,13 @@ __device__ __forceinline__ bool next_segment(Cut &c, const CutArgs &a, int x, bo
     }
     return false;
 }
-// The first segment of workgroup x of nx.  `equal` (out): all lengths are the same and every
-// sequence takes the same number of workgroups, which then leave no segment cut.  len_lane:
-// seq_lens[lane], read by the caller.
+// The first segment of workgroup x of nx.  `alone` (out): every sequence has workgroups of its own, so
+// this one has no further segment.  len_lane: seq_lens[lane], read by the caller.
 __device__ __forceinline__ bool first_segment(Cut &c, const CutArgs &a, int nx, int x, int lane, int len_lane,
-                                              bool &equal) {
+                                              bool &alone) {
     const int32_t *sl = a.seq_lens;
-    const int len0 = __builtin_amdgcn_readfirstlane(len_lane);
     uint32_t total = 0, most = 0, w0 = 0, s0 = 0;  // (w0, s0: the first 64 sequences' weights and their scan)
     int l0 = 0;
-    bool same = true;
     for (int c0 = 0; c0 < a.batch; c0 += kWave) {
         const int len = c0 + lane >= a.batch ? 0 : c0 == 0 ? len_lane : sl[c0 + lane];
         const int t = tiles_of(len);
@@ -91,7 +88,6 @@ __device__ __forceinline__ bool first_segment(Cut &c, const CutArgs &a, int nx, 
         }
         total += (uint32_t)__builtin_amdgcn_readlane((int)sc, kWave - 1);
         most = max(most, wave_max((uint32_t)t));
-        same = same && __ballot(c0 + lane < a.batch && len != len0) == 0;
     }
     if (most == 0)
         return false;
@@ -100,21 +96,23 @@ __device__ __forceinline__ bool first_segment(Cut &c, const CutArgs &a, int nx, 
     // at most num_splits parts: a sequence of T tiles touches at most (T - 1) / cell + 2 cells
     if ((uint64_t)cell * (uint32_t)(a.num_splits - 1) < most)
         cell = max(cell, (most + (uint32_t)a.num_splits - 2) / (uint32_t)(a.num_splits - 1));
-    equal = false;
-    if (same && a.per_seq > 0) {
+    alone = false;
+    if (a.per_seq > 0) {
         const int k = min(min(a.per_seq, a.num_splits), (int)div_pos((int)most + least - 1, least));
         // (3-bit keys, 48 sequences of 256 tiles on 256 workgroups: 5 each, 52 tiles, take 53.9 us;
         // stretches of 51 take 56.7)
         if ((uint32_t)div_pos((int)most + k - 1, k) <= cell + cell / 16) {
-            equal = true;
+            alone = true;
             c.b = div_pos(x, k);
             if (c.b >= a.batch)
                 return false;
-            c.len = len0;
-            c.tiles = (int)most;
+            c.len = c.b < kWave ? __builtin_amdgcn_readlane(l0, c.b) : sl[c.b];
+            c.tiles = tiles_of(c.len);
             c.p = x - c.b * k;
-            c.n_parts = k;
-            c.run = run_of(c.tiles, k, c.p);
+            c.n_parts = min(k, (int)div_pos(c.tiles + least - 1, least));
+            if (c.p >= c.n_parts)
+                return false;
+            c.run = run_of(c.tiles, c.n_parts, c.p);
             return true;
         }
     }

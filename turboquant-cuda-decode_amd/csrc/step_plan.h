@@ -22,7 +22,7 @@ constexpr int kMinWaveTiles = 4;  // a wave's stream is whole turns of the 4-slo
 struct StepPlan {
     int vw, sw;    // head parts per workgroup, waves per head part
     int nx;        // workgroups along the list of sequences
-    int per_seq;   // of them per sequence when lengths are equal
+    int per_seq;   // of them per sequence (0: fewer than one)
     bool whole;    // one workgroup per sequence, which writes the output rows itself
     // Its workgroups rotate a 16-bit query themselves.  Every segment stages all 64 KB of rot_t, 16
     // columns per wave at a time: with one or two waves that is eight or four rounds of load, barrier
