@@ -97,3 +97,14 @@ def test_uneven_batches_are_cut_into_stretches(batch, lo, hi):
     p = host.plan(batch, 8, up(hi, 16), 32)
     assert not p.whole
     assert max(len(host.segments(lens, 32, p, x)) for x in range(p.nx)) > 1
+
+
+@pytest.mark.parametrize("batch,nvh,tokens,whole", [
+    (200, 8, 500, True), (200, 8, 2000, False), (135, 8, 350, True), (135, 8, 700, False), (220, 8, 1000, True),
+    (128, 8, 500, False), (400, 4, 700, True), (520, 8, 600, True), (520, 4, 600, True), (520, 4, 1500, False), (300, 8, 300, True),
+    (256, 6, 700, True), (256, 6, 4000, False)])
+def test_batches_past_half_a_round_stay_whole_for_small_tables(batch, nvh, tokens, whole):
+    """One wave per head part: a second segment and the merge cost more than even stretches gain."""
+    p = host.plan(batch, nvh, up(tokens, 16), 32)
+    assert p.whole == whole
+    assert not whole or p.sw == 1
