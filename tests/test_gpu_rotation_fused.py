@@ -113,3 +113,20 @@ def test_fp32_queries_keep_the_rotation_launch(dev):
     torch.cuda.synchronize()
     assert not torch.isnan(ws.q_rot).any(), "fp32 queries go through the rotation launch"
     assert np.array_equal(out.cpu().numpy(), ref_out.cpu().numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("batch", [3, 256])  # the rotation inside the step, in parts and whole
+def test_rotation_matrices_need_no_more_than_float_alignment(dev, batch):
+    rng, w, query, rot_t = _case(850, max(batch, 4), 8, 4, 2000 if batch == 3 else 300)
+    t = lambda a: to_dev(a, dev)  # noqa: E731
+    q, cache, bt, sl, cents = t(query).half(), t(w.kv_cache), t(w.block_table), t(w.seq_lens), t(w.centroids)
+    room = torch.zeros(D * D + 4, dtype=torch.float32, device=dev)
+    outs = []
+    for shift in range(4):
+        r = room[shift:shift + D * D].view(D, D)
+        r.copy_(t(rot_t))
+        assert r.data_ptr() % 16 == 4 * shift
+        outs.append([x.clone() for x in ops.full_decode(q, r, cache, bt, sl, cents, 16, out_dtype=torch.float32)])
+    for out, lse in outs[1:]:
+        assert torch.equal(out.view(torch.int32), outs[0][0].view(torch.int32))
+        assert torch.equal(lse.view(torch.int32), outs[0][1].view(torch.int32))

@@ -119,13 +119,16 @@ template <int G> struct RotLoads {
     uint4 q[G / 4];
 };
 // Chunk `c` of rot_t: lane i of the workgroup's nw * 64 takes 16-byte piece i + 64 nw k of the
-// chunk's 128 rows of 4 nw pieces.
+// chunk's 128 rows of 4 nw pieces.  (rot_t is an array of floats: its pieces are 4-byte aligned.)
 template <int G>
 __device__ __forceinline__ void rot_load_pit(RotLoads<G> &r, const float *__restrict__ rot_t, int c, int nw, int tid) {
+    typedef uint32_t piece __attribute__((ext_vector_type(4), aligned(4)));
     const int per_row = 4 * nw, row = div_pos(tid, per_row), col = tid - row * per_row;  // 16 rows per load
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-        r.pit[k] = *reinterpret_cast<const uint4 *>(rot_t + (16 * k + row) * kHeadDim + 16 * nw * c + 4 * col);
+    for (int k = 0; k < 8; ++k) {
+        const piece v = *reinterpret_cast<const piece *>(rot_t + (16 * k + row) * kHeadDim + 16 * nw * c + 4 * col);
+        r.pit[k] = uint4{v[0], v[1], v[2], v[3]};
+    }
 }
 // The query rows row_base .. + n_rows - 1, 16 pieces each (n_rows <= G nw; spare lanes repeat the last piece).
 template <int G>
