@@ -83,10 +83,11 @@ def test_full_decode_random_shape(dev, c):
 
 @pytest.mark.parametrize("batch", [4, 256])
 def test_full_decode_attention_scale(dev, batch):
-    """A non-default attn_scale through both paths: the four-launch step (batch 4) and the one
-    launch with the rotation inside Stage1 (batch 256, one wave per sequence and kv-head)."""
+    """A non-default attn_scale through both forms of the step: sequences in parts with a merge
+    (batch 4, up to 5000 tokens) and whole sequences in one launch (batch 256, one wave per
+    sequence and kv-head)."""
     rng = np.random.default_rng(20261499 + batch)
-    lens = rng.integers(1, 900, batch).astype(np.int32)
+    lens = rng.integers(1, 5000 if batch == 4 else 900, batch).astype(np.int32)
     w = workloads.small(20261499 + batch, batch, lens, 16, num_q_heads=32, num_kv_heads=8)
     query = torch.from_numpy(rng.standard_normal((batch, 32, 128)).astype(np.float32)).to(torch.float16)
     rot = workloads.random_orthogonal(rng, 128)

@@ -1,14 +1,13 @@
-"""The full decode step's one-split path with the query rotation inside Stage1.
+"""The full decode step with the query rotation inside, one workgroup per sequence.
 
-When every (sequence, kv-head part) gets one wave, ``tq4_full_decode`` runs each sequence as
-one split and the Stage1 kernel writes the output rows itself; for fp16 / bf16 queries and
-Hk * parts dividing 8, the kernel also rotates the query: one workgroup per sequence holds
-its waves, which compute ``query @ rot_t`` into LDS with the rotation launch's operands and
-MFMA order.  So the step must be bit-identical to rotation launch + Stage1 (one split) +
-Stage2, run separately -- which pins the fused rotation to the rotation launch (itself
-within 2e-5 of a float64 matmul, ``test_gpu_stage2.py``) -- and within the oracle's bar.
-The fused path leaves the q_rot workspace unwritten (NaN-prefilled here), which shows
-that it ran; fp32 queries keep the rotation launch (the workspace is written).
+When one wave per (sequence, kv-head part) fills the device, ``tq4_full_decode`` gives each
+sequence one workgroup, whose waves take all its tiles and write the output rows themselves; for
+fp16 / bf16 queries they also rotate the query: together they compute ``query @ rot_t`` into LDS
+with the rotation launch's operands and MFMA order.  So the step must be bit-identical to
+rotation launch + Stage1 (one split) + Stage2, run separately -- which pins its rotation to the
+rotation launch (itself within 2e-5 of a float64 matmul, ``test_gpu_stage2.py``) -- and within
+the oracle's bar.  The step leaves the q_rot workspace unwritten (NaN-prefilled here), which
+shows that it rotated; fp32 queries keep the rotation launch (the workspace is written).
 
 Shapes: (kv-heads, GQA group) with one, two, four and eight waves per sequence, groups with
 padding heads (3, 6), two parts per kv-head (16) and four (MQA: one kv-head, 32 q-heads); rows of very large and very small
@@ -47,8 +46,8 @@ def _separate(dev, q, r, cache, bt, sl, cents, out_dtype, sinks):
     return ops.stage2(mid, sl, out_dtype=out_dtype)
 
 
-# (kv-heads, group, batch): batch * kv-heads * parts fills the device (2048 waves), so the
-# step takes the one-split path
+# (kv-heads, group, batch): batch * kv-heads * parts fills the device (2048 waves), so every
+# sequence is one workgroup's
 SHAPES = [(8, 4, 256), (8, 8, 256), (8, 3, 256), (8, 6, 256), (4, 16, 256), (4, 4, 512), (2, 8, 1024),
           (1, 8, 2048), (1, 32, 512)]
 
@@ -65,7 +64,7 @@ def test_fused_rotation_matches_the_separate_launches(dev, hk, group, batch, qdt
     out, lse = ops.full_decode(q, r, cache, bt, sl, cents, 16, out_dtype=torch.bfloat16, workspace=ws)
     ref_out, ref_lse = _separate(dev, q, r, cache, bt, sl, cents, torch.bfloat16, None)
     torch.cuda.synchronize()
-    assert torch.isnan(ws.q_rot).all(), "the one-split step rotated inside Stage1"
+    assert torch.isnan(ws.q_rot).all(), "the step left the rotation to its launch"
     a, b = out.float().cpu().numpy(), ref_out.float().cpu().numpy()
     assert np.array_equal(a, b, equal_nan=True), "fused rotation differs from the rotation launch"
     assert np.array_equal(lse.cpu().numpy(), ref_lse.cpu().numpy())

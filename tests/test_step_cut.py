@@ -9,6 +9,7 @@ import random
 import pytest
 
 import step_cut_host as host
+import test_gpu_parts as parts
 
 
 def up(a, b):
@@ -108,3 +109,35 @@ def test_batches_past_half_a_round_stay_whole_for_small_tables(batch, nvh, token
     p = host.plan(batch, nvh, up(tokens, 16), 32)
     assert p.whole == whole
     assert not whole or p.sw == 1
+
+
+def form(lens, splits, hk, group, block, whole_lines, blocks=0):
+    nvh = hk * (1 if group <= 4 else up(group, 8))
+    p = host.plan(len(lens), nvh, max(blocks, 1, up(max(lens), block)), splits, block_size=block,
+                  whole_lines=whole_lines)
+    cut = [host.segments(lens, splits, p, x) for x in range(p.nx)]
+    return dict(whole=p.whole, vw=p.vw, sw=p.sw, rotates=p.rotates, segs=max(len(c) for c in cut),
+                parts=max((s[4] for c in cut for s in c), default=0),
+                wave_tiles=max((up(s[2] - s[1], p.sw) for c in cut for s in c), default=0))
+
+
+@pytest.mark.parametrize("name", parts.CASES)
+def test_gpu_cases_take_the_form_they_name(name):
+    lens, splits, hk, group, block, layout, blocks, expected = parts.CASES[name]
+    got = form(lens, splits, hk, group, block, layout == "soa", blocks)
+    assert {k: got[k] for k in expected} == expected
+
+
+@pytest.mark.parametrize("layout,hk,group,bs,lens,expected", parts.PRESET_CASES)
+def test_gpu_preset_cases_take_the_form_they_name(layout, hk, group, bs, lens, expected):
+    if expected is not None:
+        got = form(lens, 16, hk, group, bs, False)
+        assert {k: got[k] for k in expected} == expected
+
+
+def test_gpu_sink_and_nan_cases_run_in_parts():
+    got = form(parts.SINK_LENS, 32, 8, 4, 16, True)
+    assert not got["whole"] and got["parts"] > 1
+    for lens, splits, _ in parts.NAN_CASES:
+        got = form(lens, splits, 8, 4, 16, True)
+        assert not got["whole"] and got["parts"] == min(splits, 6)
