@@ -141,3 +141,13 @@ def test_gpu_sink_and_nan_cases_run_in_parts():
     for lens, splits, _ in parts.NAN_CASES:
         got = form(lens, splits, 8, 4, 16, True)
         assert not got["whole"] and got["parts"] == min(splits, 6)
+
+
+@pytest.mark.parametrize("batch,hk,lo,hi", [(12, 2, 888, 14213), (3, 1, 93, 1500), (16, 1, 312, 5000), (24, 2, 94, 1500)])
+def test_a_segment_costs_every_wave_of_a_head_part(batch, hk, lo, hi):
+    """Workgroups of several waves per head part: a second segment takes as long as with one wave, in which
+    they do as many times the tiles, so a stretch is worth cutting short of the next sequence."""
+    lens = [lo + (hi - lo) * i // (batch - 1) for i in range(batch)]
+    p = host.plan(batch, hk, up(hi, 16), 32)
+    assert not p.whole and p.sw > 1
+    assert max(len(host.segments(lens, 32, p, x)) for x in range(p.nx)) == 1

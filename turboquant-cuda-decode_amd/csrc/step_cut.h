@@ -28,9 +28,9 @@ __device__ __forceinline__ Run run_of(int tiles, int n, int i) {
     return Run{i * q + min(i, r), q + (i < r ? 1 : 0)};
 }
 
-// One workgroup's stretch of the list.  Sequences with tiles count tiles + kSegmentTiles; the
+// One workgroup's stretch of the list.  Sequences with tiles count tiles + kSegmentTiles sw; the
 // workgroup takes [x cell, (x + 1) cell) of that weight, and of sequence b, whose weight starts
-// at `start`, the tiles that fall in it after the first kSegmentTiles.
+// at `start`, the tiles that fall in it after the first kSegmentTiles sw.
 struct Cut {
     int b;           // current sequence (its batch index); >= batch: done
     int len, tiles;
@@ -40,11 +40,13 @@ struct Cut {
     int p, n_parts;  // its part and the sequence's parts
 };
 __device__ __forceinline__ int tiles_of(int len) { return (max(len, 0) + 15) >> 4; }
-__device__ __forceinline__ uint32_t weight_of(int tiles) { return tiles > 0 ? (uint32_t)(tiles + kSegmentTiles) : 0u; }
+__device__ __forceinline__ uint32_t weight_of(int tiles, int sw) {
+    return tiles > 0 ? (uint32_t)(tiles + kSegmentTiles * sw) : 0u;
+}
 // Places the stretch in sequence c.b (c.len, c.start set).
-__device__ __forceinline__ void place(Cut &c, int x) {
+__device__ __forceinline__ void place(Cut &c, int x, int sw) {
     c.tiles = tiles_of(c.len);
-    const int64_t first = (int64_t)c.start + kSegmentTiles, lo = (int64_t)x * c.cell - first;
+    const int64_t first = (int64_t)c.start + kSegmentTiles * sw, lo = (int64_t)x * c.cell - first;
     const int t0 = (int)max(lo, (int64_t)0), t1 = (int)min(lo + (int64_t)c.cell, (int64_t)c.tiles);
     c.run = Run{t0, max(t1 - t0, 0)};
     if (c.run.count > 0) {
@@ -58,13 +60,13 @@ __device__ __forceinline__ bool next_segment(Cut &c, const CutArgs &a, int x, bo
     const uint64_t end = (uint64_t)(x + 1) * c.cell;
     while (c.b < a.batch) {
         if (inside) {  // leave sequence b
-            c.start += weight_of(tiles_of(c.len));
+            c.start += weight_of(tiles_of(c.len), a.sw);
             if (++c.b >= a.batch || c.start >= end)
                 return false;
             c.len = a.seq_lens[c.b];
         }
         inside = true;
-        place(c, x);
+        place(c, x, a.sw);
         if (c.run.count > 0)
             return true;
     }
@@ -80,7 +82,7 @@ __device__ __forceinline__ bool first_segment(Cut &c, const CutArgs &a, int nx, 
     for (int c0 = 0; c0 < a.batch; c0 += kWave) {
         const int len = c0 + lane >= a.batch ? 0 : c0 == 0 ? len_lane : sl[c0 + lane];
         const int t = tiles_of(len);
-        const uint32_t w = weight_of(t), sc = wave_scan(w);
+        const uint32_t w = weight_of(t, a.sw), sc = wave_scan(w);
         if (c0 == 0) {
             l0 = len;
             w0 = w;
@@ -127,7 +129,7 @@ __device__ __forceinline__ bool first_segment(Cut &c, const CutArgs &a, int nx, 
         uint32_t w = w0, sc = s0;
         if (c0 > 0) {
             len = c0 + lane < a.batch ? sl[c0 + lane] : 0;
-            w = weight_of(tiles_of(len));
+            w = weight_of(tiles_of(len), a.sw);
             sc = wave_scan(w);
         }
         const uint32_t before = carry + sc - w;

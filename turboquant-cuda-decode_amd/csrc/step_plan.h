@@ -8,9 +8,12 @@ namespace tq4 {
 namespace xdl {
 
 constexpr int kStepWaves = 8;  // waves per workgroup at most: two per SIMD of one CU
-// What a further segment costs a workgroup (block table, query, first loads), in tiles of its
-// stretch: a sequence counts this many tiles more than it has when the list is cut.  Measured,
-// 64 sequences of 512 to 8192 tokens, with 3 / 6 / 10 / 14 / 20: 79.7 / 78.1 / 76.3 / 75.3 / 77.3 us.
+// What a further segment costs a workgroup (block table, query, rotation, first loads), in tiles of
+// each of its waves: a sequence counts this many tiles times the waves per head part more than it has
+// when the list is cut.  Measured with one wave, 64 sequences of 512 to 8192 tokens, with 3 / 6 / 10 /
+// 14 / 20: 79.7 / 78.1 / 76.3 / 75.3 / 77.3 us; over 130 ragged batches with more waves, 7 / 10 / 14 / 20
+// relative: 1.016 / 1.007 / 1 / 1.001 (14 tiles whatever the waves: 16 sequences of 500 to 8000 tokens on
+// 1 kv-head, eight waves, 28.3 / 17.5 us, 12 of 94 to 1500 27.8 / 16.9).
 constexpr int kSegmentTiles = 14;
 // Tiles whose block-table entries a wave keeps in LDS: a stream this long runs without a stop (a
 // stop, the block-table read and the refill of the ring, costs about 3 us).
