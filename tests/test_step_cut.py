@@ -103,6 +103,7 @@ def test_uneven_batches_are_cut_into_stretches(batch, lo, hi):
 @pytest.mark.parametrize("batch,nvh,tokens,whole", [
     (200, 8, 500, True), (200, 8, 2000, False), (135, 8, 350, True), (135, 8, 700, False), (220, 8, 1000, True),
     (128, 8, 500, False), (400, 4, 700, True), (520, 8, 600, True), (520, 4, 600, True), (520, 4, 1500, False), (300, 8, 300, True),
+    (400, 8, 1000, False),
     (256, 6, 700, True), (256, 6, 4000, False)])
 def test_batches_past_half_a_round_stay_whole_for_small_tables(batch, nvh, tokens, whole):
     """One wave per head part: a second segment and the merge cost more than even stretches gain."""

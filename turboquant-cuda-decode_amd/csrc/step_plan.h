@@ -72,16 +72,16 @@ inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     const int64_t rounds = (pairs + held - 1) / held;
     const bool full = 10 * pairs >= 9 * rounds * held;
     // or the pairs fill more than half of the rounds' waves and the table holds few tiles: at most 124
-    // times the share less 32, and 40 from the second round on (its sequences start as the first ones
-    // end).  Idle waves leave the others faster, so what parts gain by even stretches has to pay for
+    // times the share less 32, or 40 with more than one round (the next one's sequences start as the
+    // first ones end).  Idle waves leave the others faster, so what parts gain by even stretches has to pay for
     // their further segments and the merge.  Whole / parts for ragged lengths (a 16th to the longest),
     // 32 / 8 heads: 200 sequences (0.78 of a round) of up to 500 tokens 29.1 / 37.0 us, 700 36.2 / 41.4,
     // 1000 51.6 / 50.2, 2000 92.5 / 74.2; 135 (0.53) 500 29.0 / 29.4, 700 35.8 / 31.6; 160 (0.63) 700
-    // 35.9 / 35.3; 300 (0.59 of two) 500 46.8 / 49.3, 700 58.9 / 56.4; 32 / 4 heads, 400 (0.78) 1000
-    // 54.7 / 62.2, 520 (0.51 of two) 600 47.5 / 61.5.  Equal lengths gain more (200 x 1000 56.8 / 64.4;
+    // 35.9 / 35.3; 300 (0.59 of two) 500 46.8 / 49.3, 700 58.9 / 56.4; 400 (0.78 of two) 1000 91.6 / 85.0;
+    // 32 / 4 heads, 400 (0.78) 1000 54.7 / 62.2, 520 (0.51 of two) 600 47.5 / 61.5.  Equal lengths gain more (200 x 1000 56.8 / 64.4;
     // 200 x 2000, beyond the line, 102.2 / 114.6).
     const bool few_tiles = 2 * pairs > rounds * held &&
-                           ((tiles + 32) * rounds * held <= 124 * pairs || (rounds > 1 && tiles <= 40));
+                           (rounds == 1 ? (tiles + 32) * held <= 124 * pairs : tiles <= 40);
     int sw = full ? 1 : floor_pow2(held / pairs, kStepWaves);
     const int64_t wave_tiles = (tiles + sw - 1) / sw;
     const int64_t parts_tiles = std::max<int64_t>(kMinWaveTiles, (pairs * tiles + held - 1) / held);
