@@ -212,8 +212,8 @@ def test_backend_decode_entry(dev, layout):
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_full_decode_fused_one_split_path(dev, out_dtype):
-    """B256 x 8 kv-heads: one wave per (sequence, kv-head), so the full step runs one split
-    per sequence and the Stage1 kernel writes the output rows itself.  Bit-identical to
+    """B256 x 8 kv-heads: one wave per (sequence, kv-head), so the full step gives each sequence
+    one workgroup, which writes the output rows itself.  Bit-identical to
     Stage1 with one split + Stage2 (including empty sequences: NaN rows, -inf LSE) and
     within the oracle's fp32 gate plus the output type's rounding."""
     rng = np.random.default_rng(207)

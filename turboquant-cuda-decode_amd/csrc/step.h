@@ -5,11 +5,13 @@
 // The tile arithmetic is stage1_xdl.h's.  What differs from its kernel is how the work is cut:
 // nobody but the merge reads the rows, so there are no splits.  A workgroup of vw * sw waves
 // covers vw consecutive head parts (waves vi) with sw waves each (sub), which take consecutive
-// runs of the workgroup's 16-token tiles and join their results in LDS.  The tiles of all
-// sequences form one list, and workgroup x of the nx along the list takes an equal stretch of
-// it, across sequence ends if need be (a segment per sequence), so ragged batches and batch
-// sizes that do not divide the device keep every CU busy to the end.  The cut is worked out
-// in the kernel from seq_lens (step_cut.h); the grid depends on shapes alone (step_plan.h).
+// runs of the workgroup's 16-token tiles and join their results in LDS.  The plan (step_plan.h)
+// either gives every sequence one workgroup, or makes one list of the tiles of all sequences, of
+// which workgroup x of the nx along it takes an equal stretch, across sequence ends if need be (a
+// segment per sequence), so that ragged batches and batch sizes that do not divide the device keep
+// the CUs about equally busy; where that ends no later, sequences get workgroups of their own.
+// The cut is worked out in the kernel from seq_lens (step_cut.h); the grid depends on shapes alone.
+// With one workgroup per sequence the longest sequence sets the time.
 //
 // Against num_splits rows of 129 floats per head this drops the mid_o traffic of all but one
 // row per workgroup, the split ends inside the stream, and for lengths that are not a multiple
@@ -17,9 +19,9 @@
 // rotation launch it saves that launch (5 to 7 us at any size: staging 64 KB of rot_t).
 //
 // Measured, full step, before (rotation, Stage1 over the splits, Stage2; 256 sequences: one
-// launch) and now: 64 x 4096 tokens with 32 / 8 heads 82.8 -> 66.3 us, AoS 97.2 -> 81.0, 64 of 512 to
-// 8192 tokens 97.1 -> 75.5, 256 x 2048 114.5 -> 114.7, one of 32768 tokens 37.4 -> 24.1 (on the GPU 38.5
-// -> 18), 3-bit 48 x 4096 64.1 -> 53.8, FP8 keys with 64 heads, 24 of 1001 to 6001, 51.7 -> 42.2.
+// launch) and now: 64 x 4096 tokens with 32 / 8 heads 83.1 -> 67.0 us, AoS 97.6 -> 81.9, 64 of 512 to
+// 8192 tokens 96.8 -> 76.0, 256 x 2048 116.8 -> 116.6, one of 32768 tokens 37.4 -> 19.4 (kernels 38.5 ->
+// 17.1 and merge 4.8), 3-bit 48 x 4096 64.9 -> 53.8, FP8 keys with 64 heads, 24 of 1001 to 6001, 51.5 -> 41.1.
 // What bounds it at these sizes is the tile loop's own issue and latency chain
 // (stage1_xdl_kernel); first loads go out 4 us and the first four tiles are done 13 us after the
 // launch starts, with every CU asking at once.
@@ -162,25 +164,25 @@ __device__ __forceinline__ void rot_store_query(const RotLoads<G> &r, unsigned c
     typedef InT in8 __attribute__((ext_vector_type(8)));
 #pragma unroll
     for (int k = 0; k < G / 4; ++k) {
-            const in8 p = __builtin_bit_cast(in8, r.q[k]);
-            float amax = 0.f;
+        const in8 p = __builtin_bit_cast(in8, r.q[k]);
+        float amax = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                amax = fmaxf(amax, fabsf(to_float<InT>(p[j])));
-            amax = row16_max(amax);
-            const int e = (amax > 0.f && amax < __builtin_inff()) ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
-            half8 h;
+        for (int j = 0; j < 8; ++j)
+            amax = fmaxf(amax, fabsf(to_float<InT>(p[j])));
+        amax = row16_max(amax);
+        const int e = (amax > 0.f && amax < __builtin_inff()) ? 15 - __builtin_amdgcn_frexp_expf(amax) : 0;
+        half8 h;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                h[j] = (_Float16)__builtin_ldexpf(to_float<InT>(p[j]), e);
-            const int i = tid + 64 * nw * k;
-            if (i < 16 * n_rows) {
-                unsigned char *row = qraw + (i >> 4) * (2 * kHeadDim + kQRawPad);
-                *reinterpret_cast<half8 *>(row + 16 * (i & 15)) = h;
-                if ((i & 15) == 0)
-                    *reinterpret_cast<int *>(row + 2 * kHeadDim) = e;
-            }
+        for (int j = 0; j < 8; ++j)
+            h[j] = (_Float16)__builtin_ldexpf(to_float<InT>(p[j]), e);
+        const int i = tid + 64 * nw * k;
+        if (i < 16 * n_rows) {
+            unsigned char *row = qraw + (i >> 4) * (2 * kHeadDim + kQRawPad);
+            *reinterpret_cast<half8 *>(row + 16 * (i & 15)) = h;
+            if ((i & 15) == 0)
+                *reinterpret_cast<int *>(row + 2 * kHeadDim) = e;
         }
+    }
 }
 // Column tile w of chunk c for every row, into the LDS rows qbuf [n_rows][kQRowFloats].  B operand
 // of step kb: rot_t rows 32kb + 8g + j, column 16w + n of the chunk, as f16 hi + lo; A operand of

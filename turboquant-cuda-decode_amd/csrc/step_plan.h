@@ -50,6 +50,9 @@ struct StepShape {
     int batch, max_blocks, block_size, num_splits;
     bool whole_lines; // a head's records are whole 128-byte lines (4-bit SoA)
 };
+// The table's width stands for the lengths, which only the device knows: under a backend's table of
+// its longest context short sequences run in parts too (one of 333 tokens, 2048 blocks: 15.0 us against
+// 12.9 under a table of 21, where separate launches take 14.6).
 inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     const int held = s.held, nvh = s.nvh;
     const int64_t pairs = (int64_t)nvh * s.batch;  // (sequence, head part) pairs
@@ -73,13 +76,13 @@ inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     const bool full = 10 * pairs >= 9 * rounds * held;
     // or the pairs fill more than half of the rounds' waves and the table holds few tiles: at most 124
     // times the share less 32, or 40 with more than one round (the next one's sequences start as the
-    // first ones end).  Idle waves leave the others faster, so what parts gain by even stretches has to pay for
-    // their further segments and the merge.  Whole / parts for ragged lengths (a 16th to the longest),
+    // first ones end).  Idle waves leave the others faster, so what parts gain by even stretches has to
+    // pay for their further segments and the merge.  Whole / parts for ragged lengths (a 16th to the longest),
     // 32 / 8 heads: 200 sequences (0.78 of a round) of up to 500 tokens 29.1 / 37.0 us, 700 36.2 / 41.4,
     // 1000 51.6 / 50.2, 2000 92.5 / 74.2; 135 (0.53) 500 29.0 / 29.4, 700 35.8 / 31.6; 160 (0.63) 700
     // 35.9 / 35.3; 300 (0.59 of two) 500 46.8 / 49.3, 700 58.9 / 56.4; 400 (0.78 of two) 1000 91.6 / 85.0;
-    // 32 / 4 heads, 400 (0.78) 1000 54.7 / 62.2, 520 (0.51 of two) 600 47.5 / 61.5.  Equal lengths gain more (200 x 1000 56.8 / 64.4;
-    // 200 x 2000, beyond the line, 102.2 / 114.6).
+    // 32 / 4 heads, 400 (0.78) 1000 54.7 / 62.2, 520 (0.51 of two) 600 47.5 / 61.5.  Equal lengths gain
+    // more (200 x 1000 56.8 / 64.4; 200 x 2000, beyond the line, 102.2 / 114.6).
     const bool few_tiles = 2 * pairs > rounds * held &&
                            (rounds == 1 ? (tiles + 32) * held <= 124 * pairs : tiles <= 40);
     int sw = full ? 1 : floor_pow2(held / pairs, kStepWaves);
@@ -89,9 +92,9 @@ inline StepPlan step_plan(const StepShape &s, bool have_parts) {
         vw = std::min(vw, kStepWaves / sw);
         return StepPlan{vw, sw, s.batch, 1, true, vw * sw >= kRotateWaves || vw == nvh};
     }
-    // parts: enough waves of a workgroup on one head part that a sequence has at most kMostParts parts to
-    // merge (and no more than there are rows); more waves than that cut ragged batches coarser
-    // (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
+    // parts: enough waves of a workgroup on one head part that sequences of equal lengths have at most
+    // kMostParts parts to merge, as far as eight waves reach (one sequence on 8 kv-heads: 32 parts); more
+    // waves than that cut ragged batches coarser (FP8 keys, 24 sequences of 1001 to 6001 tokens: 42.3 us with one wave, 44.6 with two; 64 of 512 to
     // 8192: 78.1 with one, 82.8 with two, 84.4 with four)
     constexpr int kMostParts = 16;
     sw = 1;

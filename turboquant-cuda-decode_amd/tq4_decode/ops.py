@@ -456,7 +456,7 @@ def _full_decode_preset(query, rotation_t, kv_cache, block_table, seq_lens, cent
     _require(_same_device(*tensors), "all tensors must be on the same device")
     mfma = bs >= 16 and bs & (bs - 1) == 0 and stride % 16 == 0
     if fp8 and not (mfma and query.data_ptr() % 16 == 0):
-        # the VALU kernel takes fp32 rows, and both take them aligned
+        # the VALU kernel takes fp32 rows, and both take them aligned (mfma: mfma_applies of tq4_decode.hip)
         query = ws.q_rot.copy_(query)
     rc = _lib.load().tq4_full_decode_preset(
         query.data_ptr(), DTYPES[query.dtype], None if fp8 else rotation_t.data_ptr(),
