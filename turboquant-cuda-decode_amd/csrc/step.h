@@ -258,21 +258,21 @@ __device__ __forceinline__ void put_out(void *out, int dtype, int64_t i, float v
 }
 
 // What happens to a finished segment's rows: the output itself when the workgroup held the
-// whole sequence (one row per head merges to itself: weight exp(0) = 1), else part row p.  Part 0
-// also leaves the count of parts, which tells the merge to pass over a sequence of one part.
+// whole sequence (one row per head merges to itself: weight exp(0) = 1), else part row p, and
+// from part 0 the count of parts.
 struct RowSink {
-    bool direct;      // the output itself
-    bool marked;      // a merge follows and reads the count
+    bool whole;
     int64_t row0;     // first head's row b * Hq + head
     int p, n_parts;
 };
 __device__ __forceinline__ void sink_lse(const StepArgs &a, const RowSink &s, int h, float v) {
-    float *l = part_lse(a.parts, (int64_t)a.batch * a.num_q_heads, s.row0 + h, a.num_splits);
-    if (s.direct)
+    if (s.whole) {
         a.lse[s.row0 + h] = v;
-    else
-        l[s.p] = part_lse_value(v);
-    if (s.marked && s.p == 0 && s.n_parts < a.num_splits)
+        return;
+    }
+    float *l = part_lse(a.parts, (int64_t)a.batch * a.num_q_heads, s.row0 + h, a.num_splits);
+    l[s.p] = part_lse_value(v);
+    if (s.p == 0 && s.n_parts < a.num_splits)
         l[a.num_splits - 1] = part_count_mark(s.n_parts);
 }
 // The wave's rows from registers (heads nh .. G-1 are padding).
@@ -287,7 +287,7 @@ __device__ __forceinline__ void emit_rows(const StepArgs &a, const RowSink &s, c
     for (int k = 0; k < G / 4; ++k) {
         if (h0 + k >= nh)
             continue;
-        if (s.direct) {
+        if (s.whole) {
             const int64_t r = (s.row0 + h0 + k) * kHeadDim + 8 * lc.n;
 #pragma unroll
             for (int i = 0; i < 8; ++i)
@@ -337,7 +337,7 @@ __device__ __forceinline__ void join_rows(const StepArgs &a, const RowSink &s, c
             wsum += wt;
         }
         const float inv = 1.f / wsum;
-        if (s.direct) {
+        if (s.whole) {
             const int64_t r = (s.row0 + h) * kHeadDim + 2 * lane;
             put_out(a.out, a.out_dtype, r, a0 * inv);
             put_out(a.out, a.out_dtype, r + 1, a1 * inv);
@@ -705,7 +705,7 @@ void decode_step_kernel(const StepArgs a) {
                 j += RING;
             } while (j <= last);
         }
-        const RowSink rows{a.whole || cut.n_parts == 1, !a.whole, (int64_t)b * a.num_q_heads + hb, cut.p, cut.n_parts};
+        const RowSink rows{a.whole != 0, (int64_t)b * a.num_q_heads + hb, cut.p, cut.n_parts};
         if (a.sw == 1)
             emit_rows<G, V3>(a, rows, st, acc, lc, nh);
         else
