@@ -91,13 +91,13 @@ __global__ __launch_bounds__(kWave) void stage2_kernel(const float *__restrict__
         lse[(int64_t)b * num_q_heads + h] = mx + logf(wsum);
 }
 
-// ---- Part rows: what Stage1 leaves when it runs a full decode step ----------------------
-// Inside the step nobody but the merge reads Stage1's rows, so mid_o's num_splits * 129
-// floats per (sequence, head) row hold `parts <= num_splits` rows in a layout of their own:
-// all rows' 128 outputs first (part p of row r at (r * num_splits + p) * 128), then all LSEs
-// (r * num_splits + p).  `parts` is worked out inside Stage1 (one per wave dealt to the
-// sequence); when it is below num_splits the last LSE slot, then unused, holds it as a NaN
-// with all sign, exponent and quiet bits set, which no stored LSE has.
+// ---- Part rows: what decode_step_kernel (step.h) leaves of sequences that run in parts ----
+// Nobody but the merge reads these rows, so mid_o's num_splits * 129 floats per (sequence, head) row
+// hold `parts <= num_splits` rows in a layout of their own: all rows' 128 outputs first (part p of
+// row r at (r * num_splits + p) * 128), then all LSEs (r * num_splits + p).  `parts` is worked out
+// by the kernel (one per workgroup that took tiles of the sequence); when it is below num_splits the
+// last LSE slot, then unused, holds it as a NaN with all sign, exponent and quiet bits set, which no
+// stored LSE has.
 __device__ __forceinline__ float *part_row(float *parts, int64_t row, int num_splits, int p) {
     return parts + (row * num_splits + p) * kHeadDim;
 }

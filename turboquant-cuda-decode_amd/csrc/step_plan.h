@@ -51,7 +51,7 @@ struct StepShape {
     bool whole_lines; // a head's records are whole 128-byte lines (4-bit SoA)
 };
 // The table's width stands for the lengths, which only the device knows: under a backend's table of
-// its longest context short sequences run in parts too (one of 333 tokens, 2048 blocks: 15.0 us against
+// its longest context short sequences run in parts too (one of 333 tokens, 2048 blocks: 16.1 us against
 // 12.9 under a table of 21, where separate launches take 14.6).
 inline StepPlan step_plan(const StepShape &s, bool have_parts) {
     const int held = s.held, nvh = s.nvh;
