@@ -165,8 +165,5 @@ void host_run(int tiles, int n, int i, int *first, int *count) {
     *count = r.count;
 }
 
-int host_constant(int which) {
-    const int v[] = {tq4::xdl::kStepWaves, tq4::xdl::kTableTiles, tq4::xdl::kMinWaveTiles, tq4::xdl::kSegmentTiles};
-    return v[which];
-}
+int host_waves(void) { return tq4::xdl::kStepWaves; }
 }

@@ -24,13 +24,15 @@ def lib():
     return _lib
 
 
-WAVES, TABLE_TILES, MIN_WAVE, SEGMENT = (lib().host_constant(i) for i in range(4))
+def waves():
+    """Waves per workgroup at most."""
+    return lib().host_waves()
 
 
 def plan(batch, nvh, max_blocks, splits, *, block_size=16, whole_lines=True, have_parts=True):
     """``step_plan`` on 256 CUs; ``nvh``: head parts of a sequence."""
     out = (ctypes.c_int * 6)()
-    lib().host_step_plan(CUS * WAVES, nvh, batch, max_blocks, block_size, splits, int(whole_lines),
+    lib().host_step_plan(CUS * waves(), nvh, batch, max_blocks, block_size, splits, int(whole_lines),
                          int(have_parts and splits > 1), out)
     return types.SimpleNamespace(vw=out[0], sw=out[1], nx=out[2], per_seq=out[3], whole=bool(out[4]),
                                  rotates=bool(out[5]))

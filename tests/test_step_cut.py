@@ -52,7 +52,7 @@ def test_every_tile_has_one_wave(seed):
         blocks = max(1, up(max(lens), bs)) * r.choice([1, 1, 3, 40])
         p = host.plan(batch, nvh, blocks, splits, block_size=bs, whole_lines=r.random() < 0.5,
                       have_parts=r.random() < 0.9)
-        assert nvh % p.vw == 0 and p.vw * p.sw <= host.WAVES
+        assert nvh % p.vw == 0 and p.vw * p.sw <= host.waves()
         check_cut(lens, splits, p)
 
 
